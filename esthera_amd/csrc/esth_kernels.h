@@ -603,6 +603,222 @@ __device__ __forceinline__ void esth_bitonic(float (&key)[(esth_tile<LOGM, LANES
     esth_bitonic_sizes<LOGM, 2, LANES>(key, idx, le, le / esth_tile<LOGM, LANES>::E);
 }
 
+/* ---------------------------------------------- the sort by packed keys
+ * The same network on keys packed with their positions into one double each:
+ * a compare-exchange is then v_max_f64 + v_min_f64 (5 cycles each) instead of
+ * a compare and four selects (4.5 each), and no position travels beside its
+ * key.  The double's bits, from the top: 0, the key's bits mapped to an
+ * unsigned integer of the same order (32), a tag (1), the position before
+ * the sort (in the rest); as positive doubles they order like integers.  The
+ * tag is set before each stage to 1 for the upper position of a pair and 0
+ * for the lower one: the network's swap of equal keys in descending segments,
+ * and only there, is exactly the order by (key, current position).
+ *
+ * Strides inside a lane's E positions are exchanged in registers, strides
+ * over the lowest two lane bits by DPP, and for wider ones the lanes trade
+ * positions through LDS so that another LOGE bits of the position are the
+ * register's (a b64 write and read per position in the wave's own order: no
+ * wait for other waves, no barrier).  Trades alone are bound by LDS (4 cycles
+ * of the CU's per wave access), DPP alone by VALU; two lane bits balance them.
+ *
+ * Bound by VALU (about 3,600 cycles a wave at 8 positions a lane, against
+ * 5,600).  2^21 keys, reads and writes of 3 to 5 us taken off: 9.3 -> 6.0 us
+ * at M = 512, 12 -> 6 at M = 1024, 7.9 -> 6.9 at M = 256. */
+__device__ __forceinline__ double esth_max_f64(double a, double b) {   /* fmax without its quieting of inputs */
+    double r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ double esth_min_f64(double a, double b) {
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+#define ESTH_SORT_TAG 0x20000000u   /* in the low word, below the key's last two bits */
+
+__device__ __forceinline__ double esth_sort_pack(float key, uint32_t pos) {
+    const uint32_t b = esth_f2u(key), u = b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);
+    return __builtin_bit_cast(double, ((uint64_t)(u >> 2) << 32) | (u << 30) | pos);
+}
+__device__ __forceinline__ float esth_sort_key(double v) {
+    const uint32_t u = (uint32_t)(__builtin_bit_cast(uint64_t, v) >> 30);
+    return esth_u2f(u ^ (uint32_t)(~((int32_t)u >> 31) | (int32_t)0x80000000u));
+}
+__device__ __forceinline__ double esth_sort_tag(double v, bool upper) {
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    return __builtin_bit_cast(double, upper ? u | ESTH_SORT_TAG : u & ~(uint64_t)ESTH_SORT_TAG);
+}
+
+/* doubles of LDS per sub-filter: its positions, one unused after every E (the
+ * lanes' stride is then odd and their accesses fall on different banks) */
+template <int LOGM, int LANES = esth_tile<LOGM>::LPS>
+__host__ __device__ constexpr int esth_sort_lds() {
+    return (1 << LOGM) + LANES;
+}
+
+/* the packed sort is taken from four positions per lane on: with two, a trade
+ * frees one bit only and the network above is faster (M = 128 on 64 lanes:
+ * 12.0 against 16.4 us for 2^21 keys; on 16 lanes 10.8 against 9.7, M = 256
+ * 13.8 against 13.4, M = 512 16.5 against 13.3, M = 1024 22.4 against 17.0,
+ * reads and writes of 3 to 5 us among them) */
+template <int LOGM, int LANES = esth_tile<LOGM>::LPS>
+__host__ __device__ constexpr bool esth_sort_packed() {
+    return esth_tile<LOGM, LANES>::E >= 4;
+}
+/* floats of LDS that a wave's sort takes (all its sub-filters together), at least `least` */
+template <int LOGM, int LANES = esth_tile<LOGM>::LPS>
+__host__ __device__ constexpr int esth_sort_floats(int least) {
+    const int n = esth_sort_packed<LOGM, LANES>() ? 2 * (ESTH_WAVE / LANES) * esth_sort_lds<LOGM, LANES>() : 0;
+    return n > least ? n : least;
+}
+
+/* where a lane's value r lies when the register's bits are [B, B + LOGE) of
+ * the position (the lane's low B bits below them, its others above):
+ * esth_sort_slot(lane) + esth_sort_step(r) */
+template <int LOGE, int B>
+__device__ __forceinline__ int esth_sort_slot(int laneg) {
+    const int e = (laneg & ((1 << B) - 1)) | ((laneg >> B) << (B + LOGE));
+    return e + (e >> LOGE);
+}
+template <int LOGE, int B>
+__host__ __device__ constexpr int esth_sort_step(int r) {
+    return (r << B) + ((r << B) >> LOGE);
+}
+
+/* from register bits [FROM, FROM + LOGE) to [TO, TO + LOGE) */
+template <int LOGE, int FROM, int TO>
+__device__ __forceinline__ void esth_sort_trade(double (&v)[1 << LOGE], double* lds, int laneg) {
+    double* wr = lds + esth_sort_slot<LOGE, FROM>(laneg);
+#pragma unroll
+    for (int r = 0; r < (1 << LOGE); ++r) wr[esth_sort_step<LOGE, FROM>(r)] = v[r];
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");   /* a wave's LDS accesses run in its order */
+    const double* rd = lds + esth_sort_slot<LOGE, TO>(laneg);
+#pragma unroll
+    for (int r = 0; r < (1 << LOGE); ++r) v[r] = rd[esth_sort_step<LOGE, TO>(r)];
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+}
+
+/* strides of register bits Q .. 0, the larger to the lower position; K >= 0:
+ * the other way round where bit K of the register index is set */
+template <int LOGE, int Q, int K>
+__device__ __forceinline__ void esth_sort_regs(double (&v)[1 << LOGE]) {
+    if constexpr (Q >= 0) {
+#pragma unroll
+        for (int r = 0; r < (1 << LOGE); ++r) {
+            if ((r >> Q) & 1) continue;
+            const double a = esth_sort_tag(v[r], false), b = esth_sort_tag(v[r + (1 << Q)], true);
+            const double hi = esth_max_f64(a, b), lo = esth_min_f64(a, b);
+            const bool up = K >= 0 && ((r >> (K >= 0 ? K : 0)) & 1);
+            v[r] = up ? lo : hi;
+            v[r + (1 << Q)] = up ? hi : lo;
+        }
+        esth_sort_regs<LOGE, Q - 1, K>(v);
+    }
+}
+
+/* a lane's values held negated (the sign bit of `neg` set) or not, as `want` asks */
+template <int E>
+__device__ __forceinline__ void esth_sort_sign(double (&v)[E], uint32_t& neg, uint32_t want) {
+    const uint64_t flip = (uint64_t)((neg ^ want) & 0x80000000u) << 32;
+#pragma unroll
+    for (int r = 0; r < E; ++r) v[r] = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, v[r]) ^ flip);
+    neg = want;
+}
+
+/* strides over lane bits Q .. 0.  The upper lane of a pair holds its values
+ * negated: both lanes then keep the larger of their own and minus the other's. */
+template <int E, int Q>
+__device__ __forceinline__ void esth_sort_lanes(double (&v)[E], int laneg, uint32_t& neg, uint32_t base) {
+    if constexpr (Q >= 0) {
+        esth_sort_sign<E>(v, neg, base ^ ((uint32_t)(laneg >> Q) << 31));
+        const uint32_t tag = ((laneg >> Q) & 1) ? ESTH_SORT_TAG : 0u;
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            const uint64_t u = __builtin_bit_cast(uint64_t, v[r]);
+            const uint32_t lo = ((uint32_t)u & ~ESTH_SORT_TAG) | tag, hi = (uint32_t)(u >> 32);
+            const uint32_t olo = (uint32_t)esth_xor_lane<(1 << Q)>((int)lo);
+            const uint32_t ohi = (uint32_t)esth_xor_lane<(1 << Q)>((int)hi);
+            const double mine = __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+            const double other = __builtin_bit_cast(double, ((uint64_t)ohi << 32) | olo);
+            asm("v_max_f64 %0, %1, -%2" : "=v"(v[r]) : "v"(mine), "v"(other));
+        }
+        esth_sort_lanes<E, Q - 1>(v, laneg, neg, base);
+    }
+}
+
+/* the merge's strides 2^TOP .. 1, the register holding bits [B, B + LOGE) */
+template <int LOGE, int TOP, int B>
+__device__ __forceinline__ void esth_sort_merge(double (&v)[1 << LOGE], double* lds, int laneg, uint32_t& neg,
+                                                uint32_t base) {
+    constexpr int NB = TOP - LOGE + 1;   /* lane bits still to go: the next window's lowest bit */
+    if constexpr (NB <= 2) {
+        if constexpr (B != 0) esth_sort_trade<LOGE, B, 0>(v, lds, laneg);
+        if constexpr (NB > 0) {
+            esth_sort_lanes<(1 << LOGE), NB - 1>(v, laneg, neg, base);
+            esth_sort_sign<(1 << LOGE)>(v, neg, base);
+        }
+        esth_sort_regs<LOGE, (NB > 0 ? LOGE - 1 : TOP), -1>(v);
+    } else {
+        esth_sort_trade<LOGE, B, NB>(v, lds, laneg);
+        esth_sort_regs<LOGE, LOGE - 1, -1>(v);
+        esth_sort_merge<LOGE, NB - 1, NB>(v, lds, laneg, neg, base);
+    }
+}
+
+/* merges of 2^K .. 2^LOGM positions.  A segment that is to ascend (bit K of
+ * the position set, a lane's bit from here on) is held negated, so that all
+ * lanes do the same. */
+template <int LOGM, int LOGE, int K>
+__device__ __forceinline__ void esth_sort_merges(double (&v)[1 << LOGE], double* lds, int laneg, uint32_t& neg) {
+    if constexpr (K <= LOGM) {
+        const uint32_t base = K < LOGM ? (uint32_t)(laneg >> (K - LOGE)) << 31 : 0u;
+        esth_sort_sign<(1 << LOGE)>(v, neg, base);
+        esth_sort_merge<LOGE, K - 1, 0>(v, lds, laneg, neg, base);
+        esth_sort_merges<LOGM, LOGE, K + 1>(v, lds, laneg, neg);
+    }
+}
+template <int LOGE, int K>
+__device__ __forceinline__ void esth_sort_small(double (&v)[1 << LOGE]) {
+    if constexpr (K < LOGE) {
+        esth_sort_regs<LOGE, K - 1, K>(v);
+        esth_sort_small<LOGE, K + 1>(v);
+    }
+}
+
+/* the sub-filter's keys sorted as esth_bitonic sorts them, idx their former
+ * positions; lds: esth_sort_lds doubles of the sub-filter's own.  A wave that
+ * holds a NaN (no order) or a -0 (equal to +0, but its own bits) runs
+ * esth_bitonic itself. */
+template <int LOGM, int LANES = esth_tile<LOGM>::LPS>
+__device__ __forceinline__ void esth_sort_keys(float (&key)[(esth_tile<LOGM, LANES>::E)],
+                                               int (&idx)[(esth_tile<LOGM, LANES>::E)], int le, double* lds) {
+    using TL = esth_tile<LOGM, LANES>;
+    constexpr int E = TL::E, LOGE = TL::LOGE;
+    static_assert(LOGE >= 1 && LOGM < 29, "two positions per lane, and room for the position below the tag");
+    constexpr int NAN_OR_NEG_ZERO = 0x23;   /* v_cmp_class: signaling, quiet, -0 */
+    bool odd = false;
+#pragma unroll
+    for (int r = 0; r < E; ++r) odd = odd || __builtin_amdgcn_classf(key[r], NAN_OR_NEG_ZERO);
+    if (__ballot(odd) != 0) {
+#pragma unroll
+        for (int r = 0; r < E; ++r) idx[r] = le + r;
+        esth_bitonic<LOGM, LANES>(key, idx, le);
+        return;
+    }
+    double v[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) v[r] = esth_sort_pack(key[r], (uint32_t)(le + r));
+    const int laneg = le / E;
+    esth_sort_small<LOGE, 1>(v);
+    uint32_t neg = 0u;
+    esth_sort_merges<LOGM, LOGE, LOGE>(v, lds, laneg, neg);
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        key[r] = esth_sort_key(v[r]);
+        idx[r] = (int)((uint32_t)__builtin_bit_cast(uint64_t, v[r]) & (uint32_t)(TL::M - 1));
+    }
+}
+
 /* ============================================================== argmax
  * reduce (reduce.cl:19-55), one work-group of 128 work-items: a strided pass
  * (the later element wins ties), then a tree (`other` wins ties).  Here the
@@ -765,10 +981,11 @@ __device__ __forceinline__ void esth_store_plane_run(float* __restrict__ st, int
     for (int r = 0; r < E; ++r) st[b + (size_t)r * stride] = v[r];
 }
 
-/* FROM_LDS: the sub-filter's weights and planes are already in LDS at `src`
- * (src[0..M) the weights, src[(1 + c) M ..) plane c, one sub-filter per
- * wave): the keys are read from there and the gather permutes there, with
- * no global reads */
+/* stage_w: this wave's LDS, esth_sort_floats (or, not FROM_LDS, at least its
+ * sub-filters' positions), 8-byte aligned.
+ * FROM_LDS: the sub-filter's weights and planes are already in LDS at `src`
+ * (src[0..M) the weights, src[(1 + c) M ..) plane c): the keys are read from
+ * there and the gather permutes there, with no global reads */
 /* v[r] to particle i0 + r * stride of plane c (a strided run: with stride
  * 64, each r is one coalesced store across the wave) */
 template <int E, int S>
@@ -793,6 +1010,7 @@ __device__ __forceinline__ void esth_sort_sub(float* __restrict__ w, const float
                                               int layout = ESTH_LAYOUT_SOA, const float* src = nullptr) {
     using TL = esth_tile<LOGM, LANES>;
     constexpr int M = TL::M, E = TL::E, LPS = TL::LPS;
+    constexpr bool PACKED = esth_sort_packed<LOGM, LANES>();
     static_assert(!FROM_LDS || M >= ESTH_WAVE, "an LDS-resident sub-filter of at least one wave's positions");
     const int lane = threadIdx.x & (ESTH_WAVE - 1);
     const int le = (lane % LPS) * E;
@@ -816,11 +1034,16 @@ __device__ __forceinline__ void esth_sort_sub(float* __restrict__ w, const float
 #pragma unroll
         for (int j = 0; j < S; ++j) esth_load_plane_run<E, S>(st_in, layout, N, j, base + le, in[j]);
     }
-#pragma unroll
-    for (int r = 0; r < E; ++r) idx[r] = le + r;
-    esth_bitonic<LOGM, LANES>(key, idx, le);
-    /* block max M_g = key of position 0 */
     const int lead = lane - (lane % LPS);
+    if constexpr (PACKED) {
+        esth_sort_keys<LOGM, LANES>(key, idx, le,
+                                    reinterpret_cast<double*>(stage_w) + (lead / LPS) * esth_sort_lds<LOGM, LANES>());
+    } else {
+#pragma unroll
+        for (int r = 0; r < E; ++r) idx[r] = le + r;
+        esth_bitonic<LOGM, LANES>(key, idx, le);
+    }
+    /* block max M_g = key of position 0 */
     const float mx = esth_shfl_idx(key[0], lead);
     /* the partial sums follow the one-wave tiling's order whatever LANES is:
      * each run of ED positions (that tiling's positions per lane) is chained
@@ -908,7 +1131,7 @@ __global__ __launch_bounds__(256) void k_sort(float* __restrict__ w, const float
     uint32_t g = wave * (ESTH_WAVE / LPS) + (uint32_t)(lane / LPS);
     const bool valid = g < G;   /* a whole sub-filter is valid or not */
     if (!valid) g = G - 1;
-    __shared__ float stage[4][ESTH_WAVE * esth_tile<LOGM>::E];
+    __shared__ __align__(16) float stage[4][esth_sort_floats<LOGM>(ESTH_WAVE * esth_tile<LOGM>::E)];
     esth_sort_sub<LOGM, S>(w, st_in, st_out, N, G, g, valid, winner, perm, t, bt_w, bt_s, part, log_w,
                            stage[threadIdx.x / ESTH_WAVE], layout);
 }
@@ -950,7 +1173,8 @@ __global__ __launch_bounds__(ESTH_WAVE * esth_ss_waves<LOGM>()) void k_sample_so
     constexpr int M = 1 << LOGM, S = T::S;
     static_assert(LOGM >= 7 && LOGM <= 10, "one work-group per sub-filter of 128..1024 particles");
     const float* __restrict__ frame = FA ? fa.v : frame_ptr;
-    __shared__ __align__(16) float sub[(1 + S) * M];   /* weights, then plane c at (1 + c) M */
+    /* weights, then plane c at (1 + c) M, then the sort's own */
+    __shared__ __align__(16) float sub[(1 + S) * M + esth_sort_floats<LOGM>(0)];
     constexpr int NT = ESTH_WAVE * esth_ss_waves<LOGM>();
     /* the next step's MTGP32 work-groups come first (the launcher adds them
      * only where a work-group has 256 threads and the LDS to hold a ring) */
@@ -987,7 +1211,7 @@ __global__ __launch_bounds__(ESTH_WAVE * esth_ss_waves<LOGM>()) void k_sample_so
     __syncthreads();
     if (threadIdx.x >= ESTH_WAVE) return;
     esth_sort_sub<LOGM, S, false, true>(w, nullptr, st_out, N, G, g, true, winner, nullptr, t, bt_w, bt_s, part,
-                                        log_w, nullptr, ESTH_LAYOUT_SOA, sub);
+                                        log_w, sub + (1 + S) * M, ESTH_LAYOUT_SOA, sub);
 }
 
 /* ============================================================= exchange */
@@ -1559,6 +1783,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     using T = esth_model_traits<MODEL>;
     constexpr int M = 1 << LOGM, S = T::S;
     static_assert(LOGM >= 9 && LOGM <= 10, "four resampling and sampling waves per sub-filter");
+    static_assert(esth_sort_floats<LOGM>(0) <= S * M, "the sort works where the resampled particles were");
     /* res: S planes of M; then the resampling's cdf (M), staged planes (S M)
      * and xl (8), whose space the sampling's weights and planes ((1 + S) M)
      * take over */
@@ -1613,7 +1838,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     __syncthreads();
     if (threadIdx.x >= ESTH_WAVE) return;
     esth_sort_sub<LOGM, S, false, true>(w, nullptr, tmp, N, G, g, true, winner_k1, nullptr, xk.t, bt_w_k1, bt_s_k1,
-                                        part_k1, log_w, nullptr, ESTH_LAYOUT_SOA, sub);
+                                        part_k1, log_w, res, ESTH_LAYOUT_SOA, sub);
 }
 
 /* =========================================================== Vose alias
@@ -2186,7 +2411,7 @@ __global__ __launch_bounds__(256) void kb_sort(const esth_bfilter* __restrict__ 
     if (wv >= nsub) return;
     const uint2 e = sub[wv];
     const esth_bfilter& f = F[e.x];
-    __shared__ float stage[4][ESTH_WAVE * esth_tile<LOGM>::E];
+    __shared__ __align__(16) float stage[4][esth_sort_floats<LOGM>(ESTH_WAVE * esth_tile<LOGM>::E)];
     esth_sort_sub<LOGM, S, true>(f.w, f.state, f.tmp, f.N, f.G, e.y, true, (float2*)f.winner, nullptr, f.t, f.bt_w,
                            f.bt_s, f.part, log_w, stage[threadIdx.x / ESTH_WAVE]);
 }
@@ -2216,7 +2441,7 @@ __attribute__((amdgpu_waves_per_eu(esth_kbss_waves_per_eu<MODEL>()))) void kb_sa
     static_assert(T::S == S, "state dimension of the model");
     constexpr int M = 1 << LOGM;
     constexpr int NT = ESTH_WAVE * esth_ss_waves<LOGM>();
-    __shared__ __align__(16) float lds[(1 + S) * M];
+    __shared__ __align__(16) float lds[(1 + S) * M + esth_sort_floats<LOGM>(0)];
     const uint2 e = sub[blockIdx.x];
     const esth_bfilter& f = F[e.x];
     const int carry = (int)(f.flags & 1u);
@@ -2248,7 +2473,7 @@ __attribute__((amdgpu_waves_per_eu(esth_kbss_waves_per_eu<MODEL>()))) void kb_sa
     __syncthreads();
     if (threadIdx.x >= ESTH_WAVE) return;
     esth_sort_sub<LOGM, S, false, true>(f.w, nullptr, f.tmp, f.N, f.G, e.y, true, (float2*)f.winner, nullptr, f.t,
-                                        f.bt_w, f.bt_s, f.part, log_w, nullptr, ESTH_LAYOUT_SOA, lds);
+                                        f.bt_w, f.bt_s, f.part, log_w, lds + (1 + S) * M, ESTH_LAYOUT_SOA, lds);
 }
 
 /* kb_sample_sort for the m = 64 class, over units of one filter's
