@@ -150,12 +150,11 @@ ESTH_HD void esth_sincosf(float x, float* sp, float* cp) {
     float hr = 0.5f * r2;
     float w = 1.0f - hr;
     float c = w + ((((1.0f - w) - hr)) + (r2 * r2) * pc);
-    int q = ((int)k) & 3;
-    float so, co;
-    if (q == 0)      { so = s;  co = c;  }
-    else if (q == 1) { so = c;  co = -s; }
-    else if (q == 2) { so = -s; co = -c; }
-    else             { so = -c; co = s;  }
+    /* quadrant q: (s, c), (c, -s), (-s, -c), (-c, s) */
+    const uint32_t q = (uint32_t)(int)k;
+    const float a = (q & 1u) ? c : s, b = (q & 1u) ? s : c;
+    const float so = esth_u2f(esth_f2u(a) ^ ((q << 30) & 0x80000000u));
+    const float co = esth_u2f(esth_f2u(b) ^ (((q + 1u) << 30) & 0x80000000u));
     *sp = so;
     *cp = co;
 }
@@ -229,11 +228,12 @@ ESTH_HD float esth_rcpf(float x) {
  * reciprocal, one square shared by both polynomials).  r is within about
  * 3 ulp of hypot(u, v), the angle within 1.2e-7 rad.  Only multiplies, fused
  * multiply-adds, min/max, compares and an integer subtract: no divide and no
- * square root, whose hardware sequences are the costly part of a likelihood. */
-ESTH_HD void esth_polar_abs(float u, float v, float* r, float* ang) {
+ * square root, whose hardware sequences are the costly part of a likelihood.
+ * mx: the longer side, d: the same but at least 1e-30 (the divisor). */
+ESTH_HD void esth_polar_sides(float u, float v, float mx, float d, float* r, float* ang) {
     const float au = fabsf(u), av = fabsf(v);
-    const float mx = fmaxf(au, av), mn = fminf(au, av);
-    const float t = mn * esth_rcpf(fmaxf(mx, 1e-30f));
+    const float mn = fminf(au, av);
+    const float t = mn * esth_rcpf(d);
     const float s = t * t;
     float a = esth_atanf_unit(t);
     a = (av > au) ? ESTH_PI_2 - a : a;
@@ -247,6 +247,18 @@ ESTH_HD void esth_polar_abs(float u, float v, float* r, float* ang) {
     q = esth_fma(q, s, ESTH_HYP_C1);
     q = esth_fma(q, s, ESTH_HYP_C0);
     *r = mx * q;
+}
+ESTH_HD void esth_polar_abs(float u, float v, float* r, float* ang) {
+    const float mx = fmaxf(fabsf(u), fabsf(v));
+    esth_polar_sides(u, v, mx, fmaxf(mx, 1e-30f), r, ang);
+}
+/* the same with the length at least 1e-30: one three-way maximum.  For a
+ * length that is subtracted from a range and squared: (z - r)^2 is the same
+ * number for every r up to 1e-30 (z itself is larger than 1e-22, or the
+ * square below the smallest subnormal). */
+ESTH_HD void esth_polar_floor(float u, float v, float* r, float* ang) {
+    const float d = fmaxf(fmaxf(fabsf(u), fabsf(v)), 1e-30f);
+    esth_polar_sides(u, v, d, d, r, ang);
 }
 
 /* wrap an angle to (-pi, pi] using a 2-part 2*pi */

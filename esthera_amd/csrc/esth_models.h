@@ -172,7 +172,7 @@ ESTH_HD void esth_unicycle_propagate(float* s, const float* z, const float* fr, 
 /* one landmark's squared range and bearing residuals, accumulated.  The
  * landmark offset is rotated by -(theta + zb): its length is the predicted
  * range and its angle the bearing residual wrapped to (-pi, pi]; only the
- * residual's square enters, so its magnitude suffices (esth_polar_abs). */
+ * residual's square enters, so its magnitude suffices (esth_polar_floor). */
 ESTH_HD void esth_unicycle_landmark(const float* lm, float x, float y, float ct, float st, float* acc_r,
                                     float* acc_b) {
     float dx = lm[0] - x;
@@ -182,7 +182,7 @@ ESTH_HD void esth_unicycle_landmark(const float* lm, float x, float y, float ct,
     float u = esth_fma(dx, C, dy * S);
     float v = esth_fma(dy, C, -(dx * S));
     float r, eb;
-    esth_polar_abs(u, v, &r, &eb);
+    esth_polar_floor(u, v, &r, &eb);
     float er = lm[2] - r;
     *acc_r = esth_fma(er, er, *acc_r);
     *acc_b = esth_fma(eb, eb, *acc_b);
@@ -491,12 +491,51 @@ ESTH_HD int esth_build_frame_impl(int model, const void* params, const void* con
     return esth_build_frame_n(model, params, control, measurement, dt, fr, ESTH_FRAME_FLOATS);
 }
 
+/* Box-Muller's radius sqrt(-2 ln u) of u in (0, 1], a multiple of 2^-23:
+ * sqrtf(-2 esth_logf(u)) and, on the device, the same bits for every such u
+ * without the parts those inputs do not need (esth_logf's subnormals, the
+ * division's and the square root's scaling): the division and the root are
+ * one Newton step each on the hardware's estimate and a correction by the
+ * exact remainder.  Bound by VALU; a pair of normals takes 225 cycles of a
+ * SIMD per wave instead of 277. */
+ESTH_HD float esth_boxmuller_radius(float u) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    /* u = m 2^e, m in (sqrt(1/2), sqrt(2)]: 0x3504f4 is the first mantissa above sqrt(2)'s */
+    const uint32_t b = esth_f2u(u), hi = (b + (0x00800000u - 0x003504f4u)) & 0xff800000u;
+    const float m = esth_u2f(b - hi + 0x3f800000u);
+    const float ef = (float)((int32_t)(hi - 0x3f800000u) >> 23);
+    const float n = m - 1.0f, d = m + 1.0f;
+    float y = __builtin_amdgcn_rcpf(d);
+    y = esth_fma(esth_fma(-d, y, 1.0f), y, y);
+    float f = n * y;
+    f = esth_fma(esth_fma(-d, f, n), y, f);
+    const float s = f * f;
+    float p = 9.09090909090909090909e-02f;            /* 1/11 */
+    p = esth_fma(p, s, 1.11111111111111111111e-01f);  /* 1/9 */
+    p = esth_fma(p, s, 1.42857142857142857143e-01f);  /* 1/7 */
+    p = esth_fma(p, s, 2.0e-01f);                     /* 1/5 */
+    p = esth_fma(p, s, 3.33333333333333333333e-01f);  /* 1/3 */
+    const float f2 = f + f;
+    const float lm = esth_fma(f2 * s, p, f2);
+    const float x = -2.0f * esth_fma(ef, ESTH_LN2_HI, esth_fma(ef, ESTH_LN2_LO, lm));
+    const float h = __builtin_amdgcn_rsqf(x);
+    float g = x * h;
+    const float hh = 0.5f * h;
+    g = esth_fma(esth_fma(-g, g, x), hh, g);
+    /* u = 1, or (from a first uniform outside [1, 2)) u <= 0 or u > 1 */
+    const bool edge = b - 1u >= 0x3f7fffffu;
+    if (__ballot(edge) != 0 && edge) g = u == 1.0f ? -0.0f : u == 0.0f ? INFINITY : NAN;
+    return g;
+#else
+    return sqrtf(-2.0f * esth_logf(u));
+#endif
+}
+
 /* Box-Muller of one uniform pair in [1,2) (pf_generic.cl:465-483):
  * u1 = 2 - x0 in (0,1], u2 = 2 - x1, r = sqrt(-2 ln u1), phi = 2 pi u2. */
 ESTH_HD void esth_boxmuller_pair(float x0, float x1, float* z0, float* z1) {
-    float u1 = 2.0f - x0;
+    const float r = esth_boxmuller_radius(2.0f - x0);
     float u2 = 2.0f - x1;
-    float r = sqrtf(-2.0f * esth_logf(u1));
     float phi = ESTH_2PI * u2;
     float sp, cp;
     esth_sincosf(phi, &sp, &cp);
