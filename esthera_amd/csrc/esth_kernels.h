@@ -1329,6 +1329,32 @@ struct esth_xch {
     int topo, dimx, dimy;
 };
 
+/* binary_search, pf_generic.cl:182-201, of a lane's E positions over 2^LOGM
+ * entries: on a power-of-two range each round halves it exactly, so its
+ * do-while runs LOGM rounds and its upper bound is the lower one plus a
+ * constant: a round is one LDS read at a constant offset, a compare, an add
+ * and a select.  Bound by the chain of LDS reads: the lane's searches run
+ * side by side (left to itself the compiler runs one after the other).  The
+ * resampling of 500 x 1024 particles of the arm 29.9 -> 26.2 us, of the 46 M
+ * particles in sub-filters of 128 of the 10,000-filter batch 424 -> 403 us. */
+template <int LOGM, int E>
+__device__ __forceinline__ void esth_search(const float* cdf, const float (&s)[E], int (&pick)[E]) {
+    const float* at[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r) at[r] = cdf;
+#pragma unroll
+    for (int k = LOGM - 1; k >= 0; --k) {
+        float c[E];
+#pragma unroll
+        for (int r = 0; r < E; ++r) c[r] = at[r][1 << k];
+        __builtin_amdgcn_sched_barrier(0);   /* all reads of a round before its first use */
+#pragma unroll
+        for (int r = 0; r < E; ++r) at[r] = c[r] > s[r] ? at[r] : at[r] + (1 << k);
+    }
+#pragma unroll
+    for (int r = 0; r < E; ++r) pick[r] = (int)(at[r] - cdf);
+}
+
 /* one sub-filter per wave (or 64/m per wave); every wave of the work-group
  * must call it (one barrier inside); cdf_w: this wave's 64*E floats of LDS;
  * recv: apply the exchange xch on the way in */
@@ -1438,24 +1464,15 @@ __device__ __forceinline__ void esth_resample_sub(float* __restrict__ st_main,
     const float u0 = rnd[base] - 1.0f;
     const float step = total / (float)M;
     int pick[E];
+    float pos[E];
+    if (systematic) {
 #pragma unroll
-    for (int r = 0; r < E; ++r) {
-        float s;
-        if (systematic) s = ((float)(laneg + LPS * r) + u0) * step;
-        else s = (uu[r] - 1.0f) * total;
-        /* binary_search, pf_generic.cl:182-201: on a power-of-two range each
-         * round halves it exactly, so its do-while runs LOGM rounds; unrolled,
-         * the E searches of a lane interleave */
-        int mn = 0, mxi = M - 1;
+        for (int r = 0; r < E; ++r) pos[r] = ((float)(laneg + LPS * r) + u0) * step;
+    } else {
 #pragma unroll
-        for (int it = 0; it < LOGM; ++it) {
-            const int cur = mn + (mxi - mn + 1) / 2;
-            const bool left = cdf[cur] > s;
-            mxi = left ? cur - 1 : mxi;
-            mn = left ? mn : cur;
-        }
-        pick[r] = mn & (M - 1);
+        for (int r = 0; r < E; ++r) pos[r] = (uu[r] - 1.0f) * total;
     }
+    esth_search<LOGM, E>(cdf, pos, pick);
     /* gather the selected particles through the cdf's LDS region, plane by
      * plane (every lane takes part; only resampled sub-filters store); unless
      * loaded early, the planes' loads are issued together, PB at a time */
@@ -1686,21 +1703,15 @@ __device__ __forceinline__ void esth_resample_sub2(float* __restrict__ st_main, 
     const float u0 = rnd[base] - 1.0f;
     const float step = total / (float)M;
     int pick[E];
+    float pos[E];
+    if (systematic) {
 #pragma unroll
-    for (int r = 0; r < E; ++r) {
-        float sv;
-        if (systematic) sv = ((float)(ob + ESTH_WAVE * r) + u0) * step;
-        else sv = (uu[r] - 1.0f) * total;
-        int mn = 0, mxi = M - 1;
+        for (int r = 0; r < E; ++r) pos[r] = ((float)(ob + ESTH_WAVE * r) + u0) * step;
+    } else {
 #pragma unroll
-        for (int it = 0; it < LOGM; ++it) {
-            const int cur = mn + (mxi - mn + 1) / 2;
-            const bool lft = cdf[cur] > sv;
-            mxi = lft ? cur - 1 : mxi;
-            mn = lft ? mn : cur;
-        }
-        pick[r] = mn & (M - 1);
+        for (int r = 0; r < E; ++r) pos[r] = (uu[r] - 1.0f) * total;
     }
+    esth_search<LOGM, E>(cdf, pos, pick);
     if constexpr (TO_LDS) {
         /* the sub-filter's next particles into res (S planes of M): the
          * selections, or, for a sub-filter the gate skips, the propagated
