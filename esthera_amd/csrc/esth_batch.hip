@@ -237,7 +237,12 @@ struct esth_batch {
     uint32_t* status[2] = {nullptr, nullptr};
     esth_mtgp_stream* streams = nullptr;
     float2 *winner = nullptr, *result = nullptr;
+    /* every filter's posterior sums and best particle, in pinned host memory
+     * that the argmax writes across the bus: an estimate is read without a
+     * copy, after one wait for the steps enqueued so far (10,000 estimates
+     * 140 -> 10 ms; the argmax launch 39 -> 47 us) */
     double* est = nullptr;
+    uint64_t waited = 0;   /* steps known to have run */
     uint32_t* top = nullptr;
     std::vector<std::pair<void*, size_t>> allocs;
     /* host */
@@ -274,6 +279,7 @@ static void batch_free(esth_batch* b) {
         hipEventDestroy(b->ev_consumed[i]);
     }
     hipEventDestroy(b->ev_fork);
+    if (b->est) hipHostFree(b->est);
     for (auto ev : b->tev) hipEventDestroy(ev);
     for (auto& a : b->allocs) esth_engine_release(b->e, a.first, a.second);
     if (b->stream) hipStreamDestroy(b->stream);
@@ -378,7 +384,6 @@ extern "C" int esth_batch_create(esth_engine* e, int n, const esth_filter_desc* 
     BA(b->bt_w, sizeof(float) * tGtot);
     BA(b->bt_s, sizeof(float) * tGtot * S);
     BA(b->result, sizeof(float2) * n);
-    BA(b->est, sizeof(double) * (4 + 2 * ESTH_MAX_STATE_DIM) * n);
     BA(b->top, sizeof(uint32_t) * 64 * n);
     BA(b->frames[0], sizeof(float) * b->frame_stride * n);
     BA(b->frames[1], sizeof(float) * b->frame_stride * n);
@@ -393,7 +398,11 @@ extern "C" int esth_batch_create(esth_engine* e, int n, const esth_filter_desc* 
         if (!fuse[class_of(b->hf[i].m)]) b->nchunks += (b->hf[i].N / 2 + ESTH_WAVE - 1) / ESTH_WAVE;
     if (b->nchunks) BA(b->d_chunks, sizeof(uint2) * b->nchunks);
 #undef BA
+    const size_t est_bytes = sizeof(double) * (4 + 2 * ESTH_MAX_STATE_DIM) * (size_t)n;
+    if (rc == ESTH_OK && hipHostMalloc((void**)&b->est, est_bytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess)
+        rc = esth_fail(ESTH_ERR_NOMEM, "batch: %zu bytes of pinned memory", est_bytes);
     if (rc != ESTH_OK) { batch_free(b); return rc; }
+    memset(b->est, 0, est_bytes);
     /* filter table, sub-filter tables, RNG streams */
     uint64_t goff = 0, tgoff = 0;
     std::vector<std::vector<uint2>> by_class(11);
@@ -439,7 +448,6 @@ extern "C" int esth_batch_create(esth_engine* e, int n, const esth_filter_desc* 
     if (err == hipSuccess) err = hipMemcpy(b->streams, hs.data(), sizeof(esth_mtgp_stream) * hs.size(), hipMemcpyHostToDevice);
     if (err == hipSuccess) err = hipMemcpy(b->status[0], st.data(), sizeof(uint32_t) * st.size(), hipMemcpyHostToDevice);
     if (err == hipSuccess) err = hipMemset(b->w, 0, sizeof(float) * b->Ntot);
-    if (err == hipSuccess) err = hipMemset(b->est, 0, sizeof(double) * (4 + 2 * ESTH_MAX_STATE_DIM) * n);
     if (err != hipSuccess) { batch_free(b); return esth_fail(ESTH_ERR_DEVICE, "batch upload: %s", hipGetErrorString(err)); }
     for (int lm = 0; lm <= 10; ++lm) {
         if (by_class[lm].empty()) continue;
@@ -761,11 +769,12 @@ extern "C" int esth_batch_use_graph(esth_batch* b, int enable) {
 
 extern "C" int esth_batch_estimate(esth_batch* b, int i, esth_estimate* out) {
     if (!b || !out || i < 0 || i >= b->n) return esth_fail(ESTH_ERR_INVALID, "batch estimate: bad filter %d", i);
-    ESTH_HIP(hipStreamSynchronize(b->stream));
+    if (b->waited != b->steps) {
+        ESTH_HIP(hipStreamSynchronize(b->stream));
+        b->waited = b->steps;
+    }
     const int S = b->S;
-    double h[4 + 2 * ESTH_MAX_STATE_DIM];
-    ESTH_HIP(hipMemcpy(h, b->est + (size_t)i * (4 + 2 * ESTH_MAX_STATE_DIM), sizeof(double) * (4 + 2 * (size_t)S),
-                       hipMemcpyDeviceToHost));
+    const double* h = b->est + (size_t)i * (4 + 2 * ESTH_MAX_STATE_DIM);
     memset(out, 0, sizeof(*out));
     out->state_dim = S;
     out->log_weight_max = h[0];
