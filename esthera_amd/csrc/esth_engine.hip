@@ -345,11 +345,11 @@ static int log2u(uint32_t m) { int k = 0; while ((1u << k) < m) ++k; return k; }
 template <int LOGM, int S>
 static void launch_sort_t(float* w, const float* st_in, float* st_out, uint32_t N, uint32_t G, float2* winner,
                           int* perm, uint32_t t, float* bt_w, float* bt_s, float* part, int log_w, int layout,
-                          hipStream_t s) {
+                          const esth_mtgp_inline& mi, hipStream_t s) {
     using TL = esth_tile<LOGM>;
     const uint64_t waves = (G + (ESTH_WAVE / TL::LPS) - 1) / (ESTH_WAVE / TL::LPS);
-    hipLaunchKernelGGL((k_sort<LOGM, S>), dim3(grid_for(waves * ESTH_WAVE, 256)), dim3(256), 0, s, w, st_in,
-                       st_out, N, G, winner, perm, t, bt_w, bt_s, part, log_w, layout);
+    hipLaunchKernelGGL((k_sort<LOGM, S>), dim3(mi.n + grid_for(waves * ESTH_WAVE, 256)), dim3(256), 0, s, w, st_in,
+                       st_out, N, G, winner, perm, t, bt_w, bt_s, part, log_w, layout, mi);
 }
 
 template <int LOGM, int S>
@@ -376,11 +376,16 @@ static void launch_resample_t(float* st_main, const float* st_tmp, const float* 
     default: return esth_fail(ESTH_ERR_INVALID, "m"); \
     }
 
+/* the sort's LDS holds an MTGP32 ring */
+bool esth_sort_carries_rng(uint32_t m) { return m >= 256; }
+
 int esth_launch_sort(int S, uint32_t m, float* w, const float* st_in, float* st_out, uint32_t N, uint32_t G,
                      float2* winner, int* perm, uint32_t t, float* bt_w, float* bt_s, float* part, int log_w,
-                     int layout, hipStream_t s) {
+                     int layout, hipStream_t s, const esth_mtgp_inline* mtgp) {
     const int lm = log2u(m);
-#define ESTH_SORT_ARGS w, st_in, st_out, N, G, winner, perm, t, bt_w, bt_s, part, log_w, layout, s
+    const esth_mtgp_inline mi = mtgp ? *mtgp : esth_mtgp_inline{};
+    if (mi.n && !esth_sort_carries_rng(m)) return esth_fail(ESTH_ERR_UNSUPPORTED, "MTGP32 work-groups ride in sorts of m >= 256");
+#define ESTH_SORT_ARGS w, st_in, st_out, N, G, winner, perm, t, bt_w, bt_s, part, log_w, layout, mi, s
     ESTH_TRY(esth_with_state_dim(S, [&](auto sv) {
         constexpr int SV = decltype(sv)::value;
         ESTH_DISPATCH_LOGM(launch_sort_t, SV, ESTH_SORT_ARGS);
@@ -642,21 +647,26 @@ static void launch_resample_argmax_t(float* st_main, const float* st_tmp, const 
                                      uint32_t G, float thr, int systematic, int log_w, const float2* winner,
                                      const float* part, const float* best_src, size_t plane_stride, uint32_t g_stride,
                                      float2* result, double* est, const esth_xch& xch, int carry, int layout,
-                                     hipStream_t s) {
+                                     const esth_mtgp_inline& mi, hipStream_t s) {
     /* two waves per sub-filter for m >= 512 where the work-group's two
      * sub-filters' CDFs and staged planes fit in 48 KB of LDS (at m = 256 in
      * the batched classes the halves were too short to pay for the barriers) */
     if constexpr (LOGM >= 9 && (1 + S) * (1 << LOGM) <= 6144) {
-        hipLaunchKernelGGL((k_resample2_argmax<LOGM, S>), dim3(1 + (G + 1) / 2), dim3(256), 0, s, st_main, st_tmp, w,
+        hipLaunchKernelGGL((k_resample2_argmax<LOGM, S>), dim3(mi.n + 1 + (G + 1) / 2), dim3(256), 0, s, st_main, st_tmp, w,
                            rnd, N, G, thr, systematic, log_w, winner, part, best_src, plane_stride, g_stride, result,
-                           est, xch, carry, layout);
+                           est, xch, carry, layout, mi);
     } else {
         using TL = esth_tile<LOGM>;
         const uint64_t waves = (G + (ESTH_WAVE / TL::LPS) - 1) / (ESTH_WAVE / TL::LPS);
-        hipLaunchKernelGGL((k_resample_argmax<LOGM, S>), dim3(1 + grid_for(waves * ESTH_WAVE, 256)), dim3(256), 0, s,
+        hipLaunchKernelGGL((k_resample_argmax<LOGM, S>), dim3(mi.n + 1 + grid_for(waves * ESTH_WAVE, 256)), dim3(256), 0, s,
                            st_main, st_tmp, w, rnd, N, G, thr, systematic, log_w, winner, part, best_src,
-                           plane_stride, g_stride, result, est, xch, carry, layout);
+                           plane_stride, g_stride, result, est, xch, carry, layout, mi);
     }
+}
+
+/* 256-thread work-groups; the one-wave alias up to four sub-filters each */
+bool esth_resample_carries_rng(int resampler, uint32_t m) {
+    return resampler != ESTH_RESAMPLE_ALIAS || (m >= ESTH_WAVE && m <= 512);
 }
 
 int esth_launch_resample_argmax(int resampler, int S, float* st_main, const float* st_tmp, float* w,
@@ -664,8 +674,9 @@ int esth_launch_resample_argmax(int resampler, int S, float* st_main, const floa
                                 const float2* winner, const float* part, const float* best_src, size_t plane_stride,
                                 uint32_t g_stride, float2* result, double* est, uint32_t t, int topo, int dimx,
                                 int dimy, const float* bt_w, const float* bt_s, uint32_t* top, int carry,
-                                int layout, hipStream_t s) {
+                                int layout, hipStream_t s, const esth_mtgp_inline* mtgp) {
     if (resampler == ESTH_RESAMPLE_ALIAS) return esth_fail(ESTH_ERR_UNSUPPORTED, "fused argmax: scan resamplers only");
+    const esth_mtgp_inline mi = mtgp ? *mtgp : esth_mtgp_inline{};
     const int lm = log2u(m);
     const int sys = resampler == ESTH_RESAMPLE_SYSTEMATIC;
     esth_xch xch{};
@@ -676,7 +687,7 @@ int esth_launch_resample_argmax(int resampler, int S, float* st_main, const floa
         }
         xch = {bt_w, bt_s, top, w, G, t, topo == ESTH_TOPO_TORUS ? 4u : 1u, topo, dimx, dimy};
     }
-#define ESTH_RA_ARGS st_main, st_tmp, w, rnd, N, G, thr, sys, log_w, winner, part, best_src, plane_stride, g_stride, result, est, xch, carry, layout, s
+#define ESTH_RA_ARGS st_main, st_tmp, w, rnd, N, G, thr, sys, log_w, winner, part, best_src, plane_stride, g_stride, result, est, xch, carry, layout, mi, s
     ESTH_TRY(esth_with_model_state_dim(S, [&](auto sv) {
         constexpr int SV = decltype(sv)::value;
         ESTH_DISPATCH_LOGM(launch_resample_argmax_t, SV, ESTH_RA_ARGS);
@@ -692,12 +703,12 @@ static void launch_alias_argmax_t(float* st_main, const float* st_tmp, const flo
                                   uint32_t G, float thr, int adaptive, int log_w, const float2* winner,
                                   const float* part, const float* best_src, size_t plane_stride, uint32_t g_stride,
                                   float2* result, double* est, const esth_xch& xch, int carry, int layout,
-                                  hipStream_t s) {
+                                  const esth_mtgp_inline& mi, hipStream_t s) {
     if constexpr (LOGM >= 6) {
         constexpr int WPB = esth_alias_wpb<LOGM>::value;
-        hipLaunchKernelGGL((k_alias_argmax_w<LOGM, S>), dim3(1 + (G + WPB - 1) / WPB), dim3(WPB * ESTH_WAVE), 0, s,
+        hipLaunchKernelGGL((k_alias_argmax_w<LOGM, S>), dim3(mi.n + 1 + (G + WPB - 1) / WPB), dim3(WPB * ESTH_WAVE), 0, s,
                            st_main, st_tmp, w, rnd, N, G, thr, adaptive, log_w, winner, part, best_src, plane_stride,
-                           g_stride, result, est, xch, carry, layout);
+                           g_stride, result, est, xch, carry, layout, mi);
     }
 }
 
@@ -705,8 +716,12 @@ int esth_launch_alias_argmax(int S, float* st_main, const float* st_tmp, float* 
                              uint32_t m, uint32_t G, float thr, int adaptive, int log_w, const float2* winner,
                              const float* part, const float* best_src, size_t plane_stride, uint32_t g_stride,
                              float2* result, double* est, uint32_t t, int topo, int dimx, int dimy, const float* bt_w,
-                             const float* bt_s, uint32_t* top, int carry, int layout, hipStream_t s) {
+                             const float* bt_s, uint32_t* top, int carry, int layout, hipStream_t s,
+                             const esth_mtgp_inline* mtgp) {
     if (m < ESTH_WAVE) return esth_fail(ESTH_ERR_UNSUPPORTED, "fused alias: m >= 64");
+    const esth_mtgp_inline mi = mtgp ? *mtgp : esth_mtgp_inline{};
+    if (mi.n && !esth_resample_carries_rng(ESTH_RESAMPLE_ALIAS, m))
+        return esth_fail(ESTH_ERR_UNSUPPORTED, "MTGP32 work-groups ride only in 256-thread resampling launches");
     const int lm = log2u(m);
     esth_xch xch{};
     if (t > 0 && topo != ESTH_TOPO_NONE) {
@@ -716,7 +731,7 @@ int esth_launch_alias_argmax(int S, float* st_main, const float* st_tmp, float* 
         }
         xch = {bt_w, bt_s, top, w, G, t, topo == ESTH_TOPO_TORUS ? 4u : 1u, topo, dimx, dimy};
     }
-#define ESTH_AA_ARGS st_main, st_tmp, w, rnd, N, G, thr, adaptive, log_w, winner, part, best_src, plane_stride, g_stride, result, est, xch, carry, layout, s
+#define ESTH_AA_ARGS st_main, st_tmp, w, rnd, N, G, thr, adaptive, log_w, winner, part, best_src, plane_stride, g_stride, result, est, xch, carry, layout, mi, s
     ESTH_TRY(esth_with_model_state_dim(S, [&](auto sv) {
         constexpr int SV = decltype(sv)::value;
         ESTH_DISPATCH_LOGM(launch_alias_argmax_t, SV, ESTH_AA_ARGS);

@@ -15,11 +15,15 @@
 #include "esth_internal.h"
 #include "esth_dispatch.h"
 
-/* MTGP32 words, two ways.  Where the step's sampling launch has 256-thread
- * work-groups (the fused sample+sort at m >= 512, or sample+weight alone),
- * the next step's words are generated by 96 extra work-groups of that
- * launch (inline): no second stream, no event.  Otherwise a block of
- * ESTH_RNG_BLOCK_DEFAULT steps' words is generated per launch on a second
+/* MTGP32 words, three ways.  Where the step's sampling launch has 256-thread
+ * work-groups (the fused sample+sort at m >= 512, or sample+weight alone) and
+ * lasts longer than they need, the next step's words are generated by 96
+ * extra work-groups of that launch (inline).  Where the step's launches
+ * together last that long (the resampling always has 256-thread work-groups),
+ * each of them carries a share of the next step's words (carried).  Neither
+ * needs a second stream or an event, whose waits cost the main stream 11 us
+ * at every block of steps.  Otherwise a block of ESTH_RNG_BLOCK_DEFAULT
+ * steps' words is generated per launch on a second
  * stream, one block ahead (at most ESTH_RNG_BLOCK steps, and fewer where two
  * blocks would pass ESTH_RNG_BLOCK_BYTES).  Longer blocks measured slower on
  * MI355X (0.1198 ms per step with 8-step blocks against 0.1151 with 1 for
@@ -61,6 +65,8 @@ struct esth_filter {
     int64_t main_block = -1;            /* block the main stream has waited for or generated */
     int64_t inline_block = -1;          /* block generated by the previous step's launch (B = 1) */
     bool inline_rng = false;            /* this filter generates its next step's words inline */
+    bool carried = false;               /* ... in shares of all the step's launches (words kept in the same blocks) */
+    uint64_t words_upto = 0;            /* carried: steps below this have their words */
     bool prefetch = true;
     bool fuse_sample_sort = false;      /* sample+weight and sort in one launch (k_sample_sort) */
     hipEvent_t ev_rng_done[2], ev_consumed[2], ev_fork;
@@ -123,6 +129,63 @@ static bool inline_rng_pays(const esth_filter* f) {
     const double sample_us = (double)f->N * (250.0 + 49.0 * L) / 5.1e13 * 1e6;
     const double mtgp_us = 0.5 * (double)(f->size / ESTH_MTGP_LARGE);
     return sample_us >= 1.25 * mtgp_us;
+}
+
+/* The step's launches that can carry MTGP32 work-groups, in stream order, and
+ * how long each lasts by itself (us, measured on MI355X: a launch's latency,
+ * the sampling's and the sort's VALU lane-instructions per particle at the
+ * rate they sustain, the resampling's bytes) */
+enum { ESTH_CARRY_SAMPLE, ESTH_CARRY_SORT, ESTH_CARRY_RESAMPLE, ESTH_CARRIERS };
+static void carriers(const esth_filter* f, bool fused_launch, double us[ESTH_CARRIERS]) {
+    const double n = (double)f->N;
+    double insts = 800.0;   /* the arms */
+    if (f->d.model == ESTH_MODEL_UNICYCLE) insts = 200.0 + 47.0 * ((const esth_unicycle_params*)f->params)->num_landmarks;
+    else if (f->d.model == ESTH_MODEL_UNICYCLE10) insts = 300.0;
+    else if (f->d.model == ESTH_MODEL_RANDOMWALK3) insts = 130.0;
+    const double sort = 340.0, per_us = 5.1e7, bytes_per_us = 4.0e6, launch = 6.0;
+    us[ESTH_CARRY_SAMPLE] = us[ESTH_CARRY_SORT] = us[ESTH_CARRY_RESAMPLE] = 0.0;
+    if (!fused_launch) {
+        us[ESTH_CARRY_SAMPLE] = launch + n * insts / per_us;
+        if (esth_sort_carries_rng(f->m)) us[ESTH_CARRY_SORT] = launch + n * sort / per_us;
+    } else if (esth_sample_sort_inline_rng(f->m)) {
+        us[ESTH_CARRY_SAMPLE] = launch + n * (insts + sort) / per_us;
+    }
+    if (esth_resample_carries_rng(f->d.resampler, f->m))
+        us[ESTH_CARRY_RESAMPLE] = (launch + n * 8.0 * (f->S + 1) / bytes_per_us) *
+                                  (f->d.resampler == ESTH_RESAMPLE_ALIAS ? 1.4 : 1.0);
+}
+/* a round beside a launch's own work: 0.65 to 0.8 us */
+static double mtgp_us(const esth_filter* f) { return 1.0 + 0.75 * (double)(f->size / ESTH_MTGP_LARGE); }
+
+/* Carried words cost what the generator's work-groups outlast their launches
+ * by, the second stream's about 5.5 us a step: carried up to 4 us of the
+ * former.  Measured (whole runs, carried against the second stream): 1024
+ * particles 1084 -> 995 us and 4096 1009 -> 924 (32 steps), 256,000 with the
+ * alias 1527 -> 1500; where the words take longer than the launches the
+ * second stream is the better one (the 2M-particle unicycle with 4 landmarks
+ * 14.7 ms against 17.8 carried, the dh6 arm 19.3 against 21.0). */
+static bool carried_rng_pays(const esth_filter* f) {
+    double us[ESTH_CARRIERS];
+    carriers(f, f->fuse_sample_sort, us);
+    return us[ESTH_CARRY_RESAMPLE] > 0.0 &&
+           mtgp_us(f) <= us[ESTH_CARRY_SAMPLE] + us[ESTH_CARRY_SORT] + us[ESTH_CARRY_RESAMPLE] + 4.0;
+}
+
+/* words of each stream that each launch generates: all in the resampling
+ * where it lasts that long, else in proportion to what the launches last */
+static void carried_shares(const esth_filter* f, bool fused_launch, uint32_t words[ESTH_CARRIERS]) {
+    double us[ESTH_CARRIERS];
+    carriers(f, fused_launch, us);
+    if (mtgp_us(f) <= us[ESTH_CARRY_RESAMPLE]) us[ESTH_CARRY_SAMPLE] = us[ESTH_CARRY_SORT] = 0.0;
+    const double sum = us[ESTH_CARRY_SAMPLE] + us[ESTH_CARRY_SORT] + us[ESTH_CARRY_RESAMPLE];
+    const uint32_t rounds = (uint32_t)(f->size / ESTH_MTGP_LARGE);
+    uint32_t left = rounds;
+    for (int i = 0; i < ESTH_CARRY_RESAMPLE; ++i) {
+        const uint32_t r = std::min(left, (uint32_t)(rounds * us[i] / sum + 0.5));
+        words[i] = r * ESTH_MTGP_LARGE;
+        left -= r;
+    }
+    words[ESTH_CARRY_RESAMPLE] = left * ESTH_MTGP_LARGE;
 }
 
 static int falloc(esth_filter* f, size_t bytes, void** p) {
@@ -188,6 +251,7 @@ extern "C" int esth_filter_create(esth_engine* e, const esth_filter_desc* d, con
         const long v = strtol(ev, nullptr, 10);
         if (v >= 1 && v <= ESTH_RNG_BLOCK) blk = (uint64_t)v;
     }
+    f->carried = !f->inline_rng && blk == ESTH_RNG_BLOCK_DEFAULT && carried_rng_pays(f);
     f->B = (int)std::max<uint64_t>(1, std::min<uint64_t>(blk, ESTH_RNG_BLOCK_BYTES / (2ull * sizeof(float) * f->words)));
     f->xstep = f->inline_rng && f->B == 1 && f->fuse_sample_sort && f->m == 512 && d->model == ESTH_MODEL_UNICYCLE &&
                d->resampler != ESTH_RESAMPLE_ALIAS && f->t > 0 &&
@@ -214,7 +278,7 @@ extern "C" int esth_filter_create(esth_engine* e, const esth_filter_desc* d, con
     FA(f->frames, sizeof(float) * ESTH_FRAME_FLOATS * ESTH_FRAME_RING);
     FA(f->winner, sizeof(float2) * f->G);
     FA(f->result, sizeof(float2));
-    FA(f->sring, sizeof(uint32_t) * ESTH_MTGP_N * (size_t)f->K * 2 * (size_t)(f->B + 1));
+    FA(f->sring, sizeof(uint32_t) * ESTH_MTGP_N * (size_t)f->K * (2 * (size_t)(f->B + 1) + ESTH_CARRIERS - 1));
     FA(f->top, sizeof(uint32_t) * 64);
 
     FA(f->streams, sizeof(esth_mtgp_stream) * (size_t)f->K);
@@ -332,6 +396,9 @@ static int launch_rng(esth_filter* f, uint64_t n, hipStream_t s) {
                             step_words(f, n), 1, s, f->B - kk, f->words, (uint64_t)f->K * ESTH_MTGP_N);
 }
 
+/* the status between carrier i's share of a step's words and the next one's */
+static uint32_t* status_between(esth_filter* f, int i) { return status_slot(f, 2, i); }
+
 /* whether step n's sampling launch can carry the next step's MTGP32
  * work-groups: one-step blocks, prefetch on, a 256-thread sampling launch
  * (the fused one at m >= 512, or sample+weight alone), and nothing already
@@ -342,21 +409,54 @@ static bool inline_step(esth_filter* f, bool fused_launch) {
     return f->ready_block != (int64_t)f->steps + 1;
 }
 
+/* MTGP32 work carried by each of a step's launches */
+struct esth_rng_work {
+    esth_mtgp_inline mi[ESTH_CARRIERS];
+};
+
+/* the carried words of step n = f->steps: its own, where they are missing
+ * (first step, after a restore, without prefetch), by a launch ahead of it,
+ * and the next step's in shares */
+static int rng_carried(esth_filter* f, bool fused_launch, esth_rng_work* work) {
+    const uint64_t n = f->steps;
+    if (f->words_upto <= n) {
+        ESTH_TRY(esth_launch_mtgp(f->e->d_params, status_at(f, n), status_at(f, n + 1), f->streams, f->K,
+                                  step_words(f, n), 1, f->stream));
+        f->words_upto = n + 1;
+    }
+    if (!f->prefetch) return ESTH_OK;
+    uint32_t words[ESTH_CARRIERS], first = 0;
+    carried_shares(f, fused_launch, words);
+    const uint32_t* in = status_at(f, n + 1);
+    for (int i = 0; i < ESTH_CARRIERS; ++i) {
+        if (!words[i]) continue;
+        uint32_t* out = first + words[i] == f->size ? status_at(f, n + 2) : status_between(f, i);
+        work->mi[i] = {f->e->d_params, in, out, f->streams, (uint32_t*)step_words(f, n + 1), esth_param_table()[3],
+                       first, words[i], f->K};
+        in = out;
+        first += words[i];
+    }
+    f->words_upto = n + 2;
+    return ESTH_OK;
+}
+
 /* RNG side of step n = f->steps, before its kernels.  At the first step of
  * a block the main stream uses the block's words generated inline by the
  * previous step's launch (already in stream order), waits for them
  * (prefetched on the RNG stream), or generates them itself (first step,
  * after a restore, without prefetch).  With `in` (inline_step) the next
- * step's words will be generated by this step's sampling launch and *mi
+ * step's words will be generated by this step's sampling launch and *work
  * receives that launch's MTGP32 work; otherwise, with prefetch on, the next
  * block is generated on the RNG stream while this one's steps run, once the
  * block before this one (whose buffer it reuses) has been consumed. */
-static int rng_before_step(esth_filter* f, bool in, esth_mtgp_inline* mi) {
+static int rng_before_step(esth_filter* f, bool in, bool fused_launch, esth_rng_work* work) {
     hipStream_t s = f->stream;
     const uint64_t n = f->steps;
     const int64_t b = (int64_t)(n / f->B);
     const int p = (int)(b & 1);
-    *mi = esth_mtgp_inline{};
+    *work = esth_rng_work{};
+    if (f->carried) return rng_carried(f, fused_launch, work);
+    esth_mtgp_inline* mi = &work->mi[ESTH_CARRY_SAMPLE];
     bool forked = false;
     if (f->main_block != b) {
         if (f->inline_block == b) {
@@ -380,6 +480,7 @@ static int rng_before_step(esth_filter* f, bool in, esth_mtgp_inline* mi) {
         mi->streams = f->streams;
         mi->out = (uint32_t*)step_words(f, n + 1);
         mi->mask = esth_param_table()[3];
+        mi->first = mi->count = 0;   /* all */
         mi->n = f->K;
         f->inline_block = b + 1;
         f->ready_block = b + 1;
@@ -397,6 +498,7 @@ static int rng_before_step(esth_filter* f, bool in, esth_mtgp_inline* mi) {
 /* after the last step of a block its buffer may be refilled */
 static int rng_after_step(esth_filter* f) {
     const uint64_t n = f->steps;
+    if (f->carried) return ESTH_OK;
     if (n % f->B == (uint64_t)(f->B - 1)) ESTH_HIP(hipEventRecord(f->ev_consumed[(n / f->B) & 1], f->stream));
     return ESTH_OK;
 }
@@ -407,7 +509,8 @@ static int rng_after_step(esth_filter* f) {
  * weights and sorts (into step n's sorted-side buffers), the second runs the
  * argmax, the exchange and the resampling from them. */
 static int enqueue_sample(esth_filter* f, uint64_t n, const float* d_frame, const float* h_frame, hipEvent_t* ev,
-                          const esth_mtgp_inline* mi) {
+                          const esth_rng_work* work) {
+    const esth_mtgp_inline* mi = &work->mi[ESTH_CARRY_SAMPLE];
     const bool timing = ev != nullptr;
     const bool all = timing && f->timing >= 2;
     hipStream_t s = f->stream;
@@ -440,13 +543,13 @@ static int enqueue_sample(esth_filter* f, uint64_t n, const float* d_frame, cons
         if (timing) ESTH_HIP(hipEventRecord(ev[2], s));
         /* block_sort (pf_generic.c:572-585) */
         ESTH_TRY(esth_launch_sort(f->S, f->m, f->w, f->state, f->tmp, N, f->G, x.winner, nullptr, f->t, x.bt_w,
-                                  x.bt_s, x.part, log_w, d.state_layout, s));
+                                  x.bt_s, x.part, log_w, d.state_layout, s, &work->mi[ESTH_CARRY_SORT]));
     }
     if (all) ESTH_HIP(hipEventRecord(ev[3], s));
     return ESTH_OK;
 }
 
-static int enqueue_resample(esth_filter* f, uint64_t n, hipEvent_t* ev) {
+static int enqueue_resample(esth_filter* f, uint64_t n, hipEvent_t* ev, const esth_mtgp_inline* mi = nullptr) {
     const bool all = ev != nullptr && f->timing >= 2;
     hipStream_t s = f->stream;
     const esth_filter_desc& d = f->d;
@@ -477,14 +580,14 @@ static int enqueue_resample(esth_filter* f, uint64_t n, hipEvent_t* ev) {
                                               bt ? x.bt_s : f->tmp, bt ? (size_t)f->G * f->t : (size_t)N,
                                               bt ? f->t : f->m, f->result, f->est, f->t, d.topology, f->dimx,
                                               f->dimy, x.bt_w, x.bt_s, f->top, d.carry_weights, d.state_layout,
-                                              s));
+                                              s, mi));
         else
             ESTH_TRY(esth_launch_resample_argmax(d.resampler, f->S, f->state, f->tmp, f->w, R + (size_t)N * f->V, N,
                                                  f->m, f->G, d.resampling_threshold, log_w, x.winner, x.part,
                                                  bt ? x.bt_s : f->tmp, bt ? (size_t)f->G * f->t : (size_t)N,
                                                  bt ? f->t : f->m, f->result, f->est, f->t, d.topology, f->dimx,
                                                  f->dimy, x.bt_w, x.bt_s, f->top, d.carry_weights,
-                                                 d.state_layout, s));
+                                                 d.state_layout, s, mi));
     } else {
         ESTH_TRY(esth_launch_resample(d.resampler, f->S, f->state, f->tmp, f->w, R + (size_t)N * f->V, N, f->m, f->G,
                                       d.resampling_threshold, d.adaptive, log_w, nullptr, d.carry_weights,
@@ -495,15 +598,16 @@ static int enqueue_resample(esth_filter* f, uint64_t n, hipEvent_t* ev) {
 }
 
 static int enqueue_step(esth_filter* f, uint64_t n, const float* d_frame, const float* h_frame, hipEvent_t* ev,
-                        const esth_mtgp_inline* mi) {
-    ESTH_TRY(enqueue_sample(f, n, d_frame, h_frame, ev, mi));
-    return enqueue_resample(f, n, ev);
+                        const esth_rng_work* work) {
+    ESTH_TRY(enqueue_sample(f, n, d_frame, h_frame, ev, work));
+    return enqueue_resample(f, n, ev, &work->mi[ESTH_CARRY_RESAMPLE]);
 }
 
 /* step n - 1's resampling, argmax and posterior, then step n's sampling and
  * sort, in one launch */
 static int enqueue_cross(esth_filter* f, uint64_t n, const float* d_frame, const float* h_frame, hipEvent_t* ev,
-                         const esth_mtgp_inline* mi) {
+                         const esth_rng_work* work) {
+    const esth_mtgp_inline* mi = &work->mi[ESTH_CARRY_SAMPLE];
     hipStream_t s = f->stream;
     const esth_filter_desc& d = f->d;
     const uint32_t N = (uint32_t)f->N;
@@ -536,14 +640,14 @@ static int flush(esth_filter* f) {
  * ESTH_GRAPH_SAMPLE its sample+weight and sort (the resampling left
  * pending), ESTH_GRAPH_CROSS the cross-step launch. */
 enum { ESTH_GRAPH_STEP = 0, ESTH_GRAPH_SAMPLE = 1, ESTH_GRAPH_CROSS = 2 };
-static int capture_graph(esth_filter* f, uint64_t n, int slot, const esth_mtgp_inline* mi, int mode,
+static int capture_graph(esth_filter* f, uint64_t n, int slot, const esth_rng_work* work, int mode,
                          hipGraphExec_t* out) {
     hipGraph_t g = nullptr;
     ESTH_HIP(hipStreamBeginCapture(f->stream, hipStreamCaptureModeThreadLocal));
     const float* dfr = f->frames + (size_t)slot * ESTH_FRAME_FLOATS;
-    int rc = mode == ESTH_GRAPH_CROSS    ? enqueue_cross(f, n, dfr, nullptr, nullptr, mi)
-             : mode == ESTH_GRAPH_SAMPLE ? enqueue_sample(f, n, dfr, nullptr, nullptr, mi)
-                                         : enqueue_step(f, n, dfr, nullptr, nullptr, mi);
+    int rc = mode == ESTH_GRAPH_CROSS    ? enqueue_cross(f, n, dfr, nullptr, nullptr, work)
+             : mode == ESTH_GRAPH_SAMPLE ? enqueue_sample(f, n, dfr, nullptr, nullptr, work)
+                                         : enqueue_step(f, n, dfr, nullptr, nullptr, work);
     hipError_t e2 = hipStreamEndCapture(f->stream, &g);
     if (rc != ESTH_OK) { if (g) hipGraphDestroy(g); return rc; }
     if (e2 != hipSuccess) return esth_fail(ESTH_ERR_DEVICE, "end capture: %s", hipGetErrorString(e2));
@@ -590,10 +694,10 @@ extern "C" int esth_filter_step(esth_filter* f, const void* control, const void*
     /* the cross-step launch: steps without per-stage timing */
     const bool cross = f->xstep && f->xstep_on && f->fuse_sample_sort && !level2;
     if (f->pending && !cross) ESTH_TRY(flush(f));
-    const bool in = inline_step(f, fused_launch);
+    const bool in = f->carried ? f->prefetch : inline_step(f, fused_launch);
     if (level2) ESTH_HIP(hipEventRecord(ev[0], f->stream));
-    esth_mtgp_inline mi;
-    ESTH_TRY(rng_before_step(f, in, &mi));
+    esth_rng_work work;
+    ESTH_TRY(rng_before_step(f, in, fused_launch, &work));
     if (f->use_graph) {
         const int mode = !cross ? ESTH_GRAPH_STEP : f->pending ? ESTH_GRAPH_CROSS : ESTH_GRAPH_SAMPLE;
         if (f->gexec[slot] && (f->gexec_inline[slot] != in || f->gexec_mode[slot] != mode)) {
@@ -601,7 +705,7 @@ extern "C" int esth_filter_step(esth_filter* f, const void* control, const void*
             f->gexec[slot] = nullptr;
         }
         if (!f->gexec[slot]) {
-            ESTH_TRY(capture_graph(f, n, slot, &mi, mode, &f->gexec[slot]));
+            ESTH_TRY(capture_graph(f, n, slot, &work, mode, &f->gexec[slot]));
             f->gexec_inline[slot] = in;
             f->gexec_mode[slot] = mode;
         }
@@ -613,12 +717,12 @@ extern "C" int esth_filter_step(esth_filter* f, const void* control, const void*
         if (cross) f->pending = true;
     } else if (cross) {
         if (f->pending)
-            ESTH_TRY(enqueue_cross(f, n, nullptr, hf, ev, &mi));
+            ESTH_TRY(enqueue_cross(f, n, nullptr, hf, ev, &work));
         else
-            ESTH_TRY(enqueue_sample(f, n, nullptr, hf, ev, &mi));
+            ESTH_TRY(enqueue_sample(f, n, nullptr, hf, ev, &work));
         f->pending = true;
     } else {
-        ESTH_TRY(enqueue_step(f, n, nullptr, hf, ev, &mi));
+        ESTH_TRY(enqueue_step(f, n, nullptr, hf, ev, &work));
     }
     ESTH_TRY(rng_after_step(f));
     f->steps++;
@@ -825,6 +929,7 @@ extern "C" int esth_filter_restore(esth_filter* f, const void* buf, size_t bytes
     f->ready_block = -1;
     f->main_block = -1;
     f->inline_block = -1;
+    f->words_upto = 0;
     return ESTH_OK;
 }
 

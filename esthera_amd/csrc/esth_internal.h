@@ -80,7 +80,9 @@ int esth_launch_step_x(int model, uint32_t m, float* tmp, float* w, const float*
                        hipStream_t s);
 int esth_launch_sort(int S, uint32_t m, float* w, const float* st_in, float* st_out, uint32_t N,
                      uint32_t G, float2* winner, int* perm, uint32_t t, float* bt_w, float* bt_s,
-                     float* part, int log_w, int layout, hipStream_t s);
+                     float* part, int log_w, int layout, hipStream_t s, const esth_mtgp_inline* mtgp = nullptr);
+/* whether that launch can carry MTGP32 work-groups */
+bool esth_sort_carries_rng(uint32_t m);
 /* sample+weight and block sort in one launch (one work-group per sub-filter,
  * the unsorted state kept in LDS); for 128 <= m <= 1024.  The propagated
  * state is stored to `state` only for sub-filters g with keep_all or
@@ -143,13 +145,16 @@ int esth_launch_resample_argmax(int resampler, int S, float* st_main, const floa
                                 const float2* winner, const float* part, const float* best_src, size_t plane_stride,
                                 uint32_t g_stride, float2* result, double* est, uint32_t t, int topo, int dimx,
                                 int dimy, const float* bt_w, const float* bt_s, uint32_t* top, int carry,
-                                int layout, hipStream_t s);
+                                int layout, hipStream_t s, const esth_mtgp_inline* mtgp = nullptr);
 /* the same with the one-wave Vose alias resampling (m >= 64) */
 int esth_launch_alias_argmax(int S, float* st_main, const float* st_tmp, float* w, const float* rnd, uint32_t N,
                              uint32_t m, uint32_t G, float thr, int adaptive, int log_w, const float2* winner,
                              const float* part, const float* best_src, size_t plane_stride, uint32_t g_stride,
                              float2* result, double* est, uint32_t t, int topo, int dimx, int dimy, const float* bt_w,
-                             const float* bt_s, uint32_t* top, int carry, int layout, hipStream_t s);
+                             const float* bt_s, uint32_t* top, int carry, int layout, hipStream_t s,
+                             const esth_mtgp_inline* mtgp = nullptr);
+/* whether those launches can carry MTGP32 work-groups */
+bool esth_resample_carries_rng(int resampler, uint32_t m);
 /* the global top t of the compact best-t buffer (all-to-all exchange) */
 int esth_launch_topt(const float* bt_w, uint32_t n, uint32_t t, uint32_t* top, hipStream_t s);
 

@@ -118,12 +118,16 @@ __device__ __forceinline__ float esth_bfly_max(float v) {
  * x[n-352+pos] before it, so the four LDS reads are issued together ahead
  * of the phase's write. */
 /* stream j of a launch, run by one 256-thread work-group; st: 800 words of
- * LDS (the 768-word ring and the two 16-word tables) */
+ * LDS (the 768-word ring and the two 16-word tables).  Of each step's words,
+ * `count` from `first` on (count 0: all), the status being that before the
+ * first of them. */
+#define ESTH_MTGP_LDS (ESTH_MTGP_LARGE + 32)
 __device__ __forceinline__ void esth_mtgp_wg(const uint32_t* __restrict__ params, uint32_t mask,
                                              const uint32_t* status_in, uint32_t* status_out,
                                              const esth_mtgp_stream* __restrict__ streams, uint32_t j,
                                              uint32_t* __restrict__ out, int float_mode, int nsteps,
-                                             uint64_t out_step, uint64_t status_step, uint32_t* st) {
+                                             uint64_t out_step, uint64_t status_step, uint32_t* st,
+                                             uint32_t first, uint32_t count) {
     uint32_t* tbl = st + ESTH_MTGP_LARGE;
     uint32_t* ttbl = tbl + 16;
     const int tid = threadIdx.x;
@@ -140,13 +144,13 @@ __device__ __forceinline__ void esth_mtgp_wg(const uint32_t* __restrict__ params
     if (tid < ESTH_MTGP_N - ESTH_MTGP_THREADS)
         st[ESTH_MTGP_LARGE - ESTH_MTGP_N + ESTH_MTGP_THREADS + tid] = gin[ESTH_MTGP_THREADS + tid];
     __syncthreads();
-    const int size = (int)sd.size;
+    const int size = (int)(count ? count : sd.size);
     /* start offsets (mod 768) of x[n-351] for the three phases */
     const int b0 = ESTH_MTGP_LARGE - ESTH_MTGP_N;          /* 417 */
     const int b1 = 4 * ESTH_MTGP_THREADS - ESTH_MTGP_N;    /* 673 */
     const int b2 = 2 * ESTH_MTGP_THREADS - ESTH_MTGP_N;    /* 161 */
     for (int step = 0; step < nsteps; ++step) {
-        uint32_t* o = out + (size_t)step * out_step + sd.out_off;
+        uint32_t* o = out + (size_t)step * out_step + sd.out_off + first;
         for (int i = 0; i < size; i += ESTH_MTGP_LARGE) {
 #pragma unroll
             for (int ph = 0; ph < 3; ++ph) {
@@ -184,22 +188,23 @@ static __global__ __launch_bounds__(256) void k_mtgp(const uint32_t* __restrict_
                                               const esth_mtgp_stream* __restrict__ streams, uint32_t nstreams,
                                               uint32_t* __restrict__ out, int float_mode, int nsteps,
                                               uint64_t out_step, uint64_t status_step) {
-    __shared__ uint32_t st[ESTH_MTGP_LARGE + 32];
+    __shared__ uint32_t st[ESTH_MTGP_LDS];
     for (uint32_t j = blockIdx.x; j < nstreams; j += gridDim.x) {
         esth_mtgp_wg(params, mask, status_in, status_out, streams, j, out, float_mode, nsteps, out_step, status_step,
-                     st);
+                     st, 0, 0);
         __syncthreads();   /* the ring and tables are reloaded for the next stream */
     }
 }
 
-/* one step of stream j for a sampling launch, kept out of line so that its
- * registers do not add to the sampling path's (a call per work-group) */
+/* one step of stream j for a step's launch, kept out of line so that its
+ * registers do not add to that launch's own (a call per work-group) */
 __device__ __noinline__ void esth_mtgp_wg_call(const esth_mtgp_inline mi, uint32_t j, uint32_t* st) {
-    esth_mtgp_wg(mi.params, mi.mask, mi.status_in, mi.status_out, mi.streams, j, mi.out, 1, 1, 0, 0, st);
+    esth_mtgp_wg(mi.params, mi.mask, mi.status_in, mi.status_out, mi.streams, j, mi.out, 1, 1, 0, 0, st, mi.first,
+                 mi.count);
 }
 
 /* the next step's words from the first mi.n work-groups of a 256-thread
- * sampling launch: true for those work-groups, which do nothing else */
+ * launch: true for those work-groups, which do nothing else */
 __device__ __forceinline__ bool esth_mtgp_inline_wg(const esth_mtgp_inline& mi, uint32_t* st) {
     if ((int)blockIdx.x >= mi.n) return false;
     esth_mtgp_wg_call(mi, blockIdx.x, st);
@@ -384,7 +389,7 @@ __global__ __launch_bounds__(256) void k_sample_weight(float* __restrict__ state
                                                        float* __restrict__ w, int carry,
                                                        const esth_mtgp_inline mi) {
     if (mi.n) {
-        __shared__ uint32_t mst[ESTH_MTGP_LARGE + 32];
+        __shared__ uint32_t mst[ESTH_MTGP_LDS];
         if (esth_mtgp_inline_wg(mi, mst)) return;
     }
     const float* __restrict__ frame = FA ? fa.v : frame_ptr;
@@ -1124,14 +1129,17 @@ __global__ __launch_bounds__(256) void k_sort(float* __restrict__ w, const float
                                               float2* __restrict__ winner, int* __restrict__ perm,
                                               uint32_t t, float* __restrict__ bt_w,
                                               float* __restrict__ bt_s, float* __restrict__ part,
-                                              int log_w, int layout) {
+                                              int log_w, int layout, const esth_mtgp_inline mi) {
     constexpr int LPS = esth_tile<LOGM>::LPS;
     const int lane = threadIdx.x & (ESTH_WAVE - 1);
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / ESTH_WAVE;
+    __shared__ __align__(16) float stage[4][esth_sort_floats<LOGM>(ESTH_WAVE * esth_tile<LOGM>::E)];
+    if constexpr (sizeof(stage) >= sizeof(uint32_t) * ESTH_MTGP_LDS) {   /* the launcher asks no other to carry words */
+        if (mi.n && esth_mtgp_inline_wg(mi, reinterpret_cast<uint32_t*>(stage))) return;
+    }
+    const uint32_t wave = ((blockIdx.x - (uint32_t)mi.n) * blockDim.x + threadIdx.x) / ESTH_WAVE;
     uint32_t g = wave * (ESTH_WAVE / LPS) + (uint32_t)(lane / LPS);
     const bool valid = g < G;   /* a whole sub-filter is valid or not */
     if (!valid) g = G - 1;
-    __shared__ __align__(16) float stage[4][esth_sort_floats<LOGM>(ESTH_WAVE * esth_tile<LOGM>::E)];
     esth_sort_sub<LOGM, S>(w, st_in, st_out, N, G, g, valid, winner, perm, t, bt_w, bt_s, part, log_w,
                            stage[threadIdx.x / ESTH_WAVE], layout);
 }
@@ -1178,7 +1186,7 @@ __global__ __launch_bounds__(ESTH_WAVE * esth_ss_waves<LOGM>()) void k_sample_so
     constexpr int NT = ESTH_WAVE * esth_ss_waves<LOGM>();
     /* the next step's MTGP32 work-groups come first (the launcher adds them
      * only where a work-group has 256 threads and the LDS to hold a ring) */
-    constexpr bool MT = NT == ESTH_MTGP_THREADS && (1 + S) * M >= ESTH_MTGP_LARGE + 32;
+    constexpr bool MT = NT == ESTH_MTGP_THREADS && (1 + S) * M >= ESTH_MTGP_LDS;
     if constexpr (MT) {
         if (mi.n && esth_mtgp_inline_wg(mi, reinterpret_cast<uint32_t*>(sub))) return;
     }
@@ -1535,8 +1543,9 @@ __global__ __launch_bounds__(256) void k_resample(float* __restrict__ st_main,
                                cdf_s[threadIdx.x / ESTH_WAVE], false, esth_xch{}, 0, nullptr, layout);
 }
 
-/* The step's argmax + posterior (work-group 0) beside the scan resampling
- * (work-groups 1..): the two read disjoint data (the argmax: winners,
+/* The step's argmax + posterior (one work-group) beside the scan resampling
+ * (the work-groups after it; the next step's MTGP32 words, where the launch
+ * carries any, in those before it): the two read disjoint data (the argmax: winners,
  * partials and the compact best-t copy of rank 0; the resampling: weights,
  * uniforms and the exchanged sorted state) and neither writes what the other
  * reads, so one launch does both and the argmax's single work-group runs in
@@ -1552,18 +1561,21 @@ __global__ __launch_bounds__(256) void k_resample_argmax(float* __restrict__ st_
                                                          const float* __restrict__ best_src, size_t plane_stride,
                                                          uint32_t g_stride, float2* __restrict__ result,
                                                          double* __restrict__ est, esth_xch xch, int carry,
-                                                         int layout) {
+                                                         int layout, const esth_mtgp_inline mi) {
     using TL = esth_tile<LOGM>;
     __shared__ float cdf_s[4][ESTH_WAVE * TL::E];
     __shared__ float2 sc[128];
     __shared__ float smax[4];
     __shared__ double sd[4 * (2 + S)];
-    if (blockIdx.x == 0) {
+    __shared__ uint32_t mst[ESTH_MTGP_LDS];
+    if (mi.n && esth_mtgp_inline_wg(mi, mst)) return;
+    const uint32_t bx = blockIdx.x - (uint32_t)mi.n;
+    if (bx == 0) {
         esth_argmax_block<S, 256>(winner, G, log_w, part, best_src, plane_stride, g_stride, result, est, sc, smax, sd);
         return;
     }
     const int lane = threadIdx.x & (ESTH_WAVE - 1);
-    const uint32_t wave = ((blockIdx.x - 1) * blockDim.x + threadIdx.x) / ESTH_WAVE;
+    const uint32_t wave = ((bx - 1) * blockDim.x + threadIdx.x) / ESTH_WAVE;
     uint32_t g = wave * (ESTH_WAVE / TL::LPS) + (uint32_t)(lane / TL::LPS);
     const bool valid = g < G;
     if (!valid) g = G - 1;
@@ -1751,7 +1763,7 @@ __global__ __launch_bounds__(256) void k_resample2_argmax(float* __restrict__ st
                                                           const float* __restrict__ best_src, size_t plane_stride,
                                                           uint32_t g_stride, float2* __restrict__ result,
                                                           double* __restrict__ est, esth_xch xch, int carry,
-                                                          int layout) {
+                                                          int layout, const esth_mtgp_inline mi) {
     constexpr int M = 1 << LOGM;
     __shared__ __align__(16) float cdf_s[2][M];
     __shared__ __align__(16) float stage_s[2][S * M];
@@ -1759,13 +1771,16 @@ __global__ __launch_bounds__(256) void k_resample2_argmax(float* __restrict__ st
     __shared__ float2 sc[128];
     __shared__ float smax[4];
     __shared__ double sd[4 * (2 + S)];
-    if (blockIdx.x == 0) {
+    static_assert(2 * M >= ESTH_MTGP_LDS, "an MTGP32 ring fits where the prefix sums go");
+    if (mi.n && esth_mtgp_inline_wg(mi, reinterpret_cast<uint32_t*>(cdf_s))) return;
+    const uint32_t bx = blockIdx.x - (uint32_t)mi.n;
+    if (bx == 0) {
         esth_argmax_block<S, 256>(winner, G, log_w, part, best_src, plane_stride, g_stride, result, est, sc, smax, sd);
         return;
     }
     const int wv = threadIdx.x / ESTH_WAVE;   /* 0..3: sub-filter wv / 2, half wv % 2 */
     const int j = wv >> 1;
-    uint32_t g = (blockIdx.x - 1) * 2u + (uint32_t)j;
+    uint32_t g = (bx - 1) * 2u + (uint32_t)j;
     const bool valid = g < G;
     if (!valid) g = G - 1;
     esth_resample_sub2<LOGM, S>(st_main, st_tmp, w, rnd, N, g, valid, thr, systematic, log_w, cdf_s[j], stage_s[j],
@@ -2369,19 +2384,24 @@ __global__ __launch_bounds__(256) void k_alias_argmax_w(float* __restrict__ st_m
                                                         const float* __restrict__ best_src, size_t plane_stride,
                                                         uint32_t g_stride, float2* __restrict__ result,
                                                         double* __restrict__ est, esth_xch xch, int carry,
-                                                        int layout) {
+                                                        int layout, const esth_mtgp_inline mi) {
     constexpr int WPB = esth_alias_wpb<LOGM>::value;
     __shared__ float lds[WPB][4 << LOGM];
     __shared__ float2 sc[128];
     __shared__ float smax[WPB];
     __shared__ double sd[WPB * (2 + S)];
-    if (blockIdx.x == 0) {
+    if constexpr (WPB * ESTH_WAVE == ESTH_MTGP_THREADS) {
+        static_assert((WPB << (LOGM + 2)) >= ESTH_MTGP_LDS, "an MTGP32 ring fits where the tables go");
+        if (mi.n && esth_mtgp_inline_wg(mi, reinterpret_cast<uint32_t*>(lds))) return;
+    }
+    const uint32_t bx = blockIdx.x - (uint32_t)mi.n;
+    if (bx == 0) {
         esth_argmax_block<S, WPB * ESTH_WAVE>(winner, G, log_w, part, best_src, plane_stride, g_stride, result, est, sc,
                                               smax, sd);
         return;
     }
     const uint32_t wv = threadIdx.x / ESTH_WAVE;
-    const uint32_t g = (blockIdx.x - 1) * WPB + wv;
+    const uint32_t g = (bx - 1) * WPB + wv;
     if (g >= G) return;
     esth_alias_wave<LOGM, S>(st_main, st_tmp, w, rnd, N, g, thr, adaptive, log_w, nullptr, nullptr, nullptr, carry,
                              layout, lds[wv], true, xch);

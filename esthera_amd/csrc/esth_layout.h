@@ -88,8 +88,9 @@ struct esth_mtgp_stream {
     uint64_t status;    /* index of its 351-word status in status_in / status_out */
 };
 
-/* the next step's MTGP32 words, generated by extra work-groups of a
- * sampling launch (one per stream, the launch's first n work-groups) */
+/* words [first, first + count) (count 0: all) of every stream of the next step, generated by
+ * extra work-groups of one of the step's launches (one per stream, the
+ * launch's first n work-groups) */
 struct esth_mtgp_inline {
     const uint32_t* params;
     const uint32_t* status_in;
@@ -97,6 +98,7 @@ struct esth_mtgp_inline {
     const struct esth_mtgp_stream* streams;
     uint32_t* out;
     uint32_t mask;
+    uint32_t first, count;   /* multiples of 768 */
     int n;          /* streams; 0: none */
 };
 

@@ -326,9 +326,10 @@ int esth_filter_set_fusion(esth_filter* f, int enable, int* active);
 /* How the filter's MTGP32 words are made: *inline_words = 1 when the next
  * step's words come from extra work-groups of the step's sampling launch
  * (chosen where the sampling hides them), 0 when they come from a second
- * stream in blocks of *block_steps steps (mtgp32-opencl.cl:186-242 per step;
- * no counterpart in the reference, which generates them before each step,
- * pf_generic.c:191-232). */
+ * stream or, where the step's launches together hide them, in shares from
+ * work-groups of those launches, and are kept in blocks of *block_steps steps
+ * (mtgp32-opencl.cl:186-242 per step; no counterpart in the reference, which
+ * generates them before each step, pf_generic.c:191-232). */
 int esth_filter_rng_mode(esth_filter* f, int* inline_words, int* block_steps);
 /* One launch per step across the step boundary: step k's resampling, argmax
  * and posterior run at the start of step k + 1's launch (each work-group
