@@ -493,12 +493,14 @@ static bool sample_sort_pays_t(int layout, int lm) {
 /* the fused launch is taken where it keeps 3 waves per SIMD resident, or as
  * many as the sampling alone.  Measured (whole steps, fused against two
  * launches): with 3-4 waves it wins even where the sampling alone keeps 5-8
- * (dh6 at m = 512 -11 %, robotarm5 and camera at 512 -8 %, unicycle at 1024
- * -9 %, randomwalk3 at 1024 -18 %: the state's round trip through HBM
- * between the two launches outweighs the occupancy), with 2 it loses or
- * ties (dh6 at 1024 +13 %, robotarm5 at 1024 even): the sort's registers
- * (E = m/64 keys, indices and gathered planes per lane) then leave too few
- * waves to hide the sampling's memory and arithmetic latency */
+ * (robotarm5 at m = 1024, 1024 sub-filters, 7.99 -> 7.49 ms for 32 steps and
+ * the read-back, 64 sub-filters 2.30 -> 1.43 ms, camera at 1024 3.93 -> 3.15,
+ * unicycle at 1024 -9 %, randomwalk3 at 1024 -18 %: the state's round trip
+ * through HBM between the two launches outweighs the occupancy), with 2 it
+ * loses or ties (dh6 at 1024, when one wave still gathered every plane,
+ * +13 %): too few waves are then left to hide the sampling's memory and
+ * arithmetic latency.  The wave that sorts holds E = m/64 keys and positions
+ * per lane and gathers its share of the planes, one at a time */
 bool esth_sample_sort_pays(int model, int layout, uint32_t m) {
     if (!esth_sample_sort_fits(m)) return false;
     const int lm = log2u(m);

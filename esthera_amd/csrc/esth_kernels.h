@@ -677,6 +677,12 @@ __host__ __device__ constexpr int esth_sort_floats(int least) {
     return n > least ? n : least;
 }
 
+/* whether the work-group's other waves stay for the planes after the sort */
+template <int LOGM, int S>
+__host__ __device__ constexpr bool esth_sort_shared() {
+    return esth_sort_packed<LOGM>();
+}
+
 /* where a lane's value r lies when the register's bits are [B, B + LOGE) of
  * the position (the lane's low B bits below them, its others above):
  * esth_sort_slot(lane) + esth_sort_step(r) */
@@ -1123,6 +1129,86 @@ __device__ __forceinline__ void esth_sort_sub(float* __restrict__ w, const float
     }
 }
 
+/* esth_sort_sub by a work-group of W waves whose sub-filter lies in LDS
+ * (src: its weights, then its planes; `order`: esth_sort_floats of LDS, for
+ * M >= 256): wave 0 sorts, and then each wave gathers, sums and writes planes
+ * of its own by the order and the weights that wave 0 leaves in `order`.  The
+ * sums' order is esth_sort_sub's.  Every wave of the work-group must call it
+ * (one barrier inside).  One wave doing all of it held a whole plane of every
+ * dimension in registers (131 for the dh6 arm, 230 for the robot arm at 1024)
+ * and its chain was the launch's tail: dh6 at m = 512 39.5 -> 36.9 us (84
+ * registers, 5 waves per SIMD instead of 3), and with 3 waves per SIMD the
+ * robot arm at m = 1024 now takes the fused launch: 14.0 + 26.1 us as two
+ * launches -> 28.3 (500 sub-filters). */
+template <int LOGM, int S, int W>
+__device__ __forceinline__ void esth_sort_group(float* __restrict__ w, float* __restrict__ st_out, uint32_t N,
+                                                uint32_t G, uint32_t g, float2* __restrict__ winner, uint32_t t,
+                                                float* __restrict__ bt_w, float* __restrict__ bt_s,
+                                                float* __restrict__ part, int log_w, const float* src, float* order) {
+    using TL = esth_tile<LOGM>;
+    constexpr int M = TL::M, E = TL::E;
+    static_assert(esth_sort_packed<LOGM>() && esth_sort_floats<LOGM>(0) >= 2 * M, "the order and the weights in the sort's LDS");
+    const int lane = threadIdx.x & (ESTH_WAVE - 1), wv = threadIdx.x / ESTH_WAVE;
+    const int le = lane * E;
+    const size_t base = (size_t)g * M;
+    int* ord = reinterpret_cast<int*>(order);
+    float* wts = order + M;
+    float* pg = part + (size_t)g * (2 + S);
+    if (wv == 0) {
+        float key[E], wt[E];
+        int idx[E];
+        esth_load_run<E>(src + le, key);
+        esth_sort_keys<LOGM>(key, idx, le, reinterpret_cast<double*>(order));
+        const float mx = esth_shfl_idx(key[0], 0);
+        float sw = 0.0f;
+#pragma unroll
+        for (int r = 0; r < E; ++r) {
+            wt[r] = log_w ? esth_expf(key[r] - esth_max_shift(mx)) : key[r];
+            sw = sw + wt[r];
+        }
+        esth_store_run<E>(wts + le, wt);
+#pragma unroll
+        for (int r = 0; r < E; r += 4) *reinterpret_cast<int4*>(ord + le + r) = make_int4(idx[r], idx[r + 1], idx[r + 2], idx[r + 3]);
+        esth_store_run<E>(w + base + le, key);
+        if (t > 0) {
+#pragma unroll
+            for (int r = 0; r < E; ++r)
+                if ((uint32_t)(le + r) < t) bt_w[(size_t)g * t + le + r] = key[r];
+        }
+        sw = esth_bfly_sum<1, ESTH_WAVE>(sw);
+        if (lane == 0) {
+            winner[g] = make_float2(key[0], (float)g);
+            pg[0] = log_w ? mx : 0.0f;
+            pg[1] = sw;
+        }
+    }
+    __syncthreads();
+    int idx[E];
+    float wt[E];
+    esth_load_run<E>(wts + le, wt);
+#pragma unroll
+    for (int r = 0; r < E; r += 4) {
+        const int4 q = *reinterpret_cast<const int4*>(ord + le + r);
+        idx[r] = q.x; idx[r + 1] = q.y; idx[r + 2] = q.z; idx[r + 3] = q.w;
+    }
+#pragma unroll 1
+    for (int c = (wv + W - 1) % W; c < S; c += W) {
+        float v[E], acc = 0.0f;
+#pragma unroll
+        for (int r = 0; r < E; ++r) v[r] = src[(1 + c) * M + idx[r]];
+#pragma unroll
+        for (int r = 0; r < E; ++r) acc = esth_fma(wt[r], v[r], acc);
+        esth_store_run<E>(st_out + (size_t)c * N + base + le, v);
+        if (t > 0) {
+#pragma unroll
+            for (int r = 0; r < E; ++r)
+                if ((uint32_t)(le + r) < t) bt_s[(size_t)c * G * t + (size_t)g * t + le + r] = v[r];
+        }
+        acc = esth_bfly_sum<1, ESTH_WAVE>(acc);
+        if (lane == 0) pg[2 + c] = acc;
+    }
+}
+
 template <int LOGM, int S>
 __global__ __launch_bounds__(256) void k_sort(float* __restrict__ w, const float* __restrict__ st_in,
                                               float* __restrict__ st_out, uint32_t N, uint32_t G,
@@ -1217,9 +1303,14 @@ __global__ __launch_bounds__(ESTH_WAVE * esth_ss_waves<LOGM>()) void k_sample_so
         for (int c = 0; c < S; ++c) *reinterpret_cast<float2*>(sub + (1 + c) * M + q) = make_float2(s0[c], s1[c]);
     }
     __syncthreads();
-    if (threadIdx.x >= ESTH_WAVE) return;
-    esth_sort_sub<LOGM, S, false, true>(w, nullptr, st_out, N, G, g, true, winner, nullptr, t, bt_w, bt_s, part,
-                                        log_w, sub + (1 + S) * M, ESTH_LAYOUT_SOA, sub);
+    if constexpr (esth_sort_shared<LOGM, S>()) {
+        esth_sort_group<LOGM, S, esth_ss_waves<LOGM>()>(w, st_out, N, G, g, winner, t, bt_w, bt_s, part, log_w, sub,
+                                                        sub + (1 + S) * M);
+    } else {
+        if (threadIdx.x >= ESTH_WAVE) return;
+        esth_sort_sub<LOGM, S, false, true>(w, nullptr, st_out, N, G, g, true, winner, nullptr, t, bt_w, bt_s, part,
+                                            log_w, sub + (1 + S) * M, ESTH_LAYOUT_SOA, sub);
+    }
 }
 
 /* ============================================================= exchange */
@@ -1862,9 +1953,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
         for (int c = 0; c < S; ++c) *reinterpret_cast<float2*>(sub + (1 + c) * M + q) = make_float2(s0[c], s1[c]);
     }
     __syncthreads();
-    if (threadIdx.x >= ESTH_WAVE) return;
-    esth_sort_sub<LOGM, S, false, true>(w, nullptr, tmp, N, G, g, true, winner_k1, nullptr, xk.t, bt_w_k1, bt_s_k1,
-                                        part_k1, log_w, res, ESTH_LAYOUT_SOA, sub);
+    if constexpr (esth_sort_shared<LOGM, S>()) {
+        esth_sort_group<LOGM, S, 4>(w, tmp, N, G, g, winner_k1, xk.t, bt_w_k1, bt_s_k1, part_k1, log_w, sub, res);
+    } else {
+        if (threadIdx.x >= ESTH_WAVE) return;
+        esth_sort_sub<LOGM, S, false, true>(w, nullptr, tmp, N, G, g, true, winner_k1, nullptr, xk.t, bt_w_k1,
+                                            bt_s_k1, part_k1, log_w, res, ESTH_LAYOUT_SOA, sub);
+    }
 }
 
 /* =========================================================== Vose alias
@@ -2502,9 +2597,14 @@ __attribute__((amdgpu_waves_per_eu(esth_kbss_waves_per_eu<MODEL>()))) void kb_sa
         for (int c = 0; c < S; ++c) *reinterpret_cast<float2*>(lds + (1 + c) * M + q) = make_float2(s0[c], s1[c]);
     }
     __syncthreads();
-    if (threadIdx.x >= ESTH_WAVE) return;
-    esth_sort_sub<LOGM, S, false, true>(f.w, nullptr, f.tmp, f.N, f.G, e.y, true, (float2*)f.winner, nullptr, f.t,
-                                        f.bt_w, f.bt_s, f.part, log_w, lds + (1 + S) * M, ESTH_LAYOUT_SOA, lds);
+    if constexpr (esth_sort_shared<LOGM, S>()) {
+        esth_sort_group<LOGM, S, esth_ss_waves<LOGM>()>(f.w, f.tmp, f.N, f.G, e.y, (float2*)f.winner, f.t, f.bt_w,
+                                                        f.bt_s, f.part, log_w, lds, lds + (1 + S) * M);
+    } else {
+        if (threadIdx.x >= ESTH_WAVE) return;
+        esth_sort_sub<LOGM, S, false, true>(f.w, nullptr, f.tmp, f.N, f.G, e.y, true, (float2*)f.winner, nullptr, f.t,
+                                            f.bt_w, f.bt_s, f.part, log_w, lds + (1 + S) * M, ESTH_LAYOUT_SOA, lds);
+    }
 }
 
 /* kb_sample_sort for the m = 64 class, over units of one filter's
