@@ -1354,44 +1354,84 @@ static __global__ void k_exchange(float* __restrict__ st, float* __restrict__ w,
     for (int c = 0; c < S; ++c) st[(size_t)c * N + dst] = bt_s[(size_t)c * Gt + src];
 }
 
-/* Global top-t of the G*t candidates by (weight desc, index asc): t rounds,
- * each selecting the best candidate strictly after the previous one. */
+/* Global top-t of n candidates by (weight desc, index asc), by one work-group
+ * of 1024: t rounds, each selecting the best candidate strictly after the
+ * previous one.  A round is one pass over the candidates (held in registers
+ * up to 8 per thread) and a tree over the 1024 threads' best: the tree's
+ * levels 512 .. 64 apart in the first wave's registers, the others by lane
+ * exchanges, two barriers a round.  Bound by latency (2000 candidates, 4
+ * rounds: 11.6 -> 9.9 us).  sw, si: 1024 words of LDS each. */
+struct esth_cand {
+    float w;
+    uint32_t i;
+};
+__device__ __forceinline__ esth_cand esth_cand_best(esth_cand a, esth_cand o) {
+    const bool take = o.i != 0xffffffffu && (a.i == 0xffffffffu || o.w > a.w || (o.w == a.w && o.i < a.i));
+    return take ? o : a;
+}
+__device__ __forceinline__ void esth_topt_block(const float* __restrict__ bt_w, uint32_t n, uint32_t t,
+                                                uint32_t* __restrict__ top, float* sw, uint32_t* si) {
+    constexpr int K = 8;
+    const int l = threadIdx.x;
+    const bool held = n <= 1024u * K;
+    float v[K];
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        const uint32_t c = (uint32_t)l + 1024u * (uint32_t)j;
+        v[j] = held && c < n ? bt_w[c] : 0.0f;
+    }
+    float pw = INFINITY;
+    uint32_t pi = 0;
+    for (uint32_t k = 0; k < t; ++k) {
+        esth_cand best{-INFINITY, 0xffffffffu};
+        auto visit = [&](float x, uint32_t c) {
+            const bool after = k == 0 || x < pw || (x == pw && c > pi);
+            const bool better = best.i == 0xffffffffu || x > best.w || (x == best.w && c < best.i);
+            if (after && better) best = esth_cand{x, c};
+        };
+        if (held) {
+#pragma unroll
+            for (int j = 0; j < K; ++j) {
+                const uint32_t c = (uint32_t)l + 1024u * (uint32_t)j;
+                if (c < n) visit(v[j], c);
+            }
+        } else {
+            for (uint32_t c = (uint32_t)l; c < n; c += 1024u) visit(bt_w[c], c);
+        }
+        sw[l] = best.w;
+        si[l] = best.i;
+        __syncthreads();
+        if (l < ESTH_WAVE) {
+            esth_cand e[16];
+#pragma unroll
+            for (int j = 0; j < 16; ++j) e[j] = esth_cand{sw[l + 64 * j], si[l + 64 * j]};
+#pragma unroll
+            for (int d = 8; d > 0; d >>= 1)
+#pragma unroll
+                for (int j = 0; j < d; ++j) e[j] = esth_cand_best(e[j], e[j + d]);
+#pragma unroll
+            for (int d = 32; d > 0; d >>= 1) {
+                const int src = (l + d) & (ESTH_WAVE - 1);
+                const esth_cand o{esth_shfl_idx(e[0].w, src), (uint32_t)__builtin_amdgcn_ds_bpermute(src << 2, (int)e[0].i)};
+                if (l < d) e[0] = esth_cand_best(e[0], o);
+            }
+            if (l == 0) {
+                sw[0] = e[0].w;
+                si[0] = e[0].i;
+                top[k] = e[0].i;
+            }
+        }
+        __syncthreads();
+        pw = sw[0];
+        pi = si[0];
+        __syncthreads();
+    }
+}
 static __global__ __launch_bounds__(1024) void k_topt(const float* __restrict__ bt_w, uint32_t n, uint32_t t,
                                                uint32_t* __restrict__ top) {
     __shared__ float sw[1024];
     __shared__ uint32_t si[1024];
-    const int l = threadIdx.x;
-    float pw = INFINITY;
-    uint32_t pi = 0;
-    bool have_prev = false;
-    for (uint32_t k = 0; k < t; ++k) {
-        float bw = -INFINITY;
-        uint32_t bi = 0xffffffffu;
-        for (uint32_t c = (uint32_t)l; c < n; c += 1024) {
-            float v = bt_w[c];
-            bool after = !have_prev || (v < pw) || (v == pw && c > pi);
-            bool better = (bi == 0xffffffffu) || (v > bw) || (v == bw && c < bi);
-            if (after && better) { bw = v; bi = c; }
-        }
-        sw[l] = bw;
-        si[l] = bi;
-        __syncthreads();
-        for (int off = 512; off > 0; off >>= 1) {
-            if (l < off) {
-                float ow = sw[l + off];
-                uint32_t oi = si[l + off];
-                bool take = (oi != 0xffffffffu) &&
-                            ((si[l] == 0xffffffffu) || ow > sw[l] || (ow == sw[l] && oi < si[l]));
-                if (take) { sw[l] = ow; si[l] = oi; }
-            }
-            __syncthreads();
-        }
-        pw = sw[0];
-        pi = si[0];
-        have_prev = true;
-        if (l == 0) top[k] = pi;
-        __syncthreads();
-    }
+    esth_topt_block(bt_w, n, t, top, sw, si);
 }
 
 /* cross-lane levels of the scan tree: lx[k] = sibling node at level k */
@@ -2687,39 +2727,7 @@ static __global__ __launch_bounds__(1024) void kb_topt(const esth_bfilter* __res
     __shared__ float sw[1024];
     __shared__ uint32_t si[1024];
     const esth_bfilter& f = F[blockIdx.x];
-    const int l = threadIdx.x;
-    const uint32_t n = f.G * f.t;
-    float pw = INFINITY;
-    uint32_t pi = 0;
-    bool have_prev = false;
-    for (uint32_t k = 0; k < f.t; ++k) {
-        float bw = -INFINITY;
-        uint32_t bi = 0xffffffffu;
-        for (uint32_t c = (uint32_t)l; c < n; c += 1024) {
-            float v = f.bt_w[c];
-            bool after = !have_prev || (v < pw) || (v == pw && c > pi);
-            bool better = (bi == 0xffffffffu) || (v > bw) || (v == bw && c < bi);
-            if (after && better) { bw = v; bi = c; }
-        }
-        sw[l] = bw;
-        si[l] = bi;
-        __syncthreads();
-        for (int off = 512; off > 0; off >>= 1) {
-            if (l < off) {
-                float ow = sw[l + off];
-                uint32_t oi = si[l + off];
-                bool take = (oi != 0xffffffffu) &&
-                            ((si[l] == 0xffffffffu) || ow > sw[l] || (ow == sw[l] && oi < si[l]));
-                if (take) { sw[l] = ow; si[l] = oi; }
-            }
-            __syncthreads();
-        }
-        pw = sw[0];
-        pi = si[0];
-        have_prev = true;
-        if (l == 0) f.top[k] = pi;
-        __syncthreads();
-    }
+    esth_topt_block(f.bt_w, f.G * f.t, f.t, f.top, sw, si);
 }
 
 /* one thread per received slot: nslots = (torus ? 4 : 1) * t slots per sub-filter */
