@@ -21,17 +21,22 @@
  * extra work-groups of that launch (inline).  Where the step's launches
  * together last that long (the resampling always has 256-thread work-groups),
  * each of them carries a share of the next step's words (carried).  Neither
- * needs a second stream or an event, whose waits cost the main stream 11 us
- * at every block of steps.  Otherwise a block of ESTH_RNG_BLOCK_DEFAULT
- * steps' words is generated per launch on a second
- * stream, one block ahead (at most ESTH_RNG_BLOCK steps, and fewer where two
- * blocks would pass ESTH_RNG_BLOCK_BYTES).  Longer blocks measured slower on
- * MI355X (0.1198 ms per step with 8-step blocks against 0.1151 with 1 for
- * the 2M-particle unicycle): one MTGP32 launch that runs for several steps
- * holds its 96 work-groups beside the sampling longer than the step's own
- * words need. */
+ * needs a second stream or an event, whose waits cost the main stream 10 us
+ * at every block of steps.  Otherwise a block of steps' words is generated
+ * per launch on a second stream, one block ahead: ESTH_RNG_BLOCK_LONG steps,
+ * or fewer where two blocks would pass ESTH_RNG_BLOCK_CACHED, but not fewer
+ * than ESTH_RNG_BLOCK_DEFAULT (nor two blocks above ESTH_RNG_BLOCK_BYTES).
+ * Whole runs with blocks of 2, 3 and 4 steps: randomwalk3 128 x 3001 (two
+ * blocks of 4: 49 MB) 2.27, -, 2.03 ms; unicycle with 4 landmarks 512 x 2048
+ * (134 MB) 9.13, 9.05, 8.93 ms; dh6 512 x 2048 (235 MB) 18.56, 18.21, 18.46;
+ * unicycle 512 x 4096 (268 MB) 14.54, 14.33, 14.93: the words of two blocks
+ * have to lie in the 256 MB Infinity Cache with what the step's launches
+ * read.  Blocks of 8 gain 1-3 % more at 128 x 3001, but a run's first step
+ * waits for a whole block. */
 #define ESTH_RNG_BLOCK 8
 #define ESTH_RNG_BLOCK_DEFAULT 2
+#define ESTH_RNG_BLOCK_LONG 4
+#define ESTH_RNG_BLOCK_CACHED (200ull << 20)
 #define ESTH_RNG_BLOCK_BYTES (1ull << 30)
 /* graph replay: one captured graph and one device frame slot per step of the
  * two word blocks */
@@ -70,6 +75,7 @@ struct esth_filter {
     bool prefetch = true;
     bool fuse_sample_sort = false;      /* sample+weight and sort in one launch (k_sample_sort) */
     hipEvent_t ev_rng_done[2], ev_consumed[2], ev_fork;
+    bool consumed[2] = {};   /* ev_consumed recorded after that parity's last block */
     float2 *winner = nullptr, *result = nullptr;
     /* the posterior sums and best particle: pinned host memory that the argmax
      * writes across the bus (4 + 2 S doubles), so that reading an estimate is
@@ -246,23 +252,32 @@ extern "C" int esth_filter_create(esth_engine* e, const esth_filter_desc* d, con
     for (int i = 0; i < ESTH_FRAME_RING; ++i) hipEventCreateWithFlags(&f->frame_ev[i], hipEventDisableTiming);
     /* ESTH_RNG_BLOCK_STEPS (1..ESTH_RNG_BLOCK) overrides the block length */
     f->inline_rng = (!f->fuse_sample_sort || esth_sample_sort_inline_rng(f->m)) && inline_rng_pays(f);
-    uint64_t blk = f->inline_rng ? 1 : ESTH_RNG_BLOCK_DEFAULT;
+    uint64_t blk = 0;
     if (const char* ev = getenv("ESTH_RNG_BLOCK_STEPS")) {
         const long v = strtol(ev, nullptr, 10);
         if (v >= 1 && v <= ESTH_RNG_BLOCK) blk = (uint64_t)v;
     }
-    f->carried = !f->inline_rng && blk == ESTH_RNG_BLOCK_DEFAULT && carried_rng_pays(f);
-    f->B = (int)std::max<uint64_t>(1, std::min<uint64_t>(blk, ESTH_RNG_BLOCK_BYTES / (2ull * sizeof(float) * f->words)));
+    f->carried = !f->inline_rng && (blk == 0 || blk == ESTH_RNG_BLOCK_DEFAULT) && carried_rng_pays(f);
+    const uint64_t two = 2ull * sizeof(float) * f->words;   /* two blocks of one step */
+    if (blk == 0)
+        blk = f->inline_rng ? 1
+              : f->carried  ? ESTH_RNG_BLOCK_DEFAULT
+                            : std::min<uint64_t>(ESTH_RNG_BLOCK_LONG,
+                                                 std::max<uint64_t>(ESTH_RNG_BLOCK_DEFAULT, ESTH_RNG_BLOCK_CACHED / two));
+    f->B = (int)std::max<uint64_t>(1, std::min<uint64_t>(blk, ESTH_RNG_BLOCK_BYTES / two));
     f->xstep = f->inline_rng && f->B == 1 && f->fuse_sample_sort && f->m == 512 && d->model == ESTH_MODEL_UNICYCLE &&
                d->resampler != ESTH_RESAMPLE_ALIAS && f->t > 0 &&
                (d->topology == ESTH_TOPO_RING || d->topology == ESTH_TOPO_TORUS) && !d->carry_weights &&
                d->state_layout == ESTH_LAYOUT_SOA;
     for (int i = 0; i < 7; ++i) hipEventCreate(&f->ev[i]);
+    /* these order launches of one device: no system-scope write-back at each
+     * (4 landmarks, 2M particles 14.83 -> 14.54 ms, dh6 18.77 -> 18.52, two
+     * events per block of 2 steps) */
     for (int i = 0; i < 2; ++i) {
-        hipEventCreateWithFlags(&f->ev_rng_done[i], hipEventDisableTiming);
-        hipEventCreateWithFlags(&f->ev_consumed[i], hipEventDisableTiming);
+        hipEventCreateWithFlags(&f->ev_rng_done[i], hipEventDisableTiming | hipEventDisableSystemFence);
+        hipEventCreateWithFlags(&f->ev_consumed[i], hipEventDisableTiming | hipEventDisableSystemFence);
     }
-    hipEventCreateWithFlags(&f->ev_fork, hipEventDisableTiming);
+    hipEventCreateWithFlags(&f->ev_fork, hipEventDisableTiming | hipEventDisableSystemFence);
     int rc = ESTH_OK;
     const size_t SN = (size_t)S * f->N;
     const size_t tG = (size_t)(f->t ? f->t : 1) * f->G;
@@ -487,7 +502,14 @@ static int rng_before_step(esth_filter* f, bool in, bool fused_launch, esth_rng_
         return ESTH_OK;
     }
     if (f->prefetch && f->ready_block != b + 1) {
-        if (!forked && b > 0) ESTH_HIP(hipStreamWaitEvent(f->rng_stream, f->ev_consumed[p ^ 1], 0));
+        if (!forked && b > 0) {
+            hipEvent_t e = f->ev_consumed[p ^ 1];
+            if (!f->consumed[p ^ 1]) {   /* the block before generated inline: everything up to here */
+                e = f->ev_fork;
+                ESTH_HIP(hipEventRecord(e, s));
+            }
+            ESTH_HIP(hipStreamWaitEvent(f->rng_stream, e, 0));
+        }
         ESTH_TRY(launch_rng(f, (uint64_t)(b + 1) * f->B, f->rng_stream));
         ESTH_HIP(hipEventRecord(f->ev_rng_done[p ^ 1], f->rng_stream));
         f->ready_block = b + 1;
@@ -495,11 +517,17 @@ static int rng_before_step(esth_filter* f, bool in, bool fused_launch, esth_rng_
     return ESTH_OK;
 }
 
-/* after the last step of a block its buffer may be refilled */
-static int rng_after_step(esth_filter* f) {
+/* after the last step of a block its buffer may be refilled.  A step that
+ * generates the next one's words inline needs no event: the refill follows
+ * on the same stream, and an event between two launches holds the second one
+ * back (the 2M-particle unicycle with 32 landmarks: 2.5 us a step, 112.5 ->
+ * 110.0) */
+static int rng_after_step(esth_filter* f, bool in) {
     const uint64_t n = f->steps;
-    if (f->carried) return ESTH_OK;
-    if (n % f->B == (uint64_t)(f->B - 1)) ESTH_HIP(hipEventRecord(f->ev_consumed[(n / f->B) & 1], f->stream));
+    if (f->carried || n % f->B != (uint64_t)(f->B - 1)) return ESTH_OK;
+    const int p = (int)((n / f->B) & 1);
+    f->consumed[p] = !in;
+    if (!in) ESTH_HIP(hipEventRecord(f->ev_consumed[p], f->stream));
     return ESTH_OK;
 }
 
@@ -724,7 +752,7 @@ extern "C" int esth_filter_step(esth_filter* f, const void* control, const void*
     } else {
         ESTH_TRY(enqueue_step(f, n, nullptr, hf, ev, &work));
     }
-    ESTH_TRY(rng_after_step(f));
+    ESTH_TRY(rng_after_step(f, in));
     f->steps++;
     return ESTH_OK;
 }
