@@ -656,7 +656,8 @@ static int batch_kernels(esth_batch* b, int p) {
 
 static int launch_rng_b(esth_batch* b, uint64_t k, hipStream_t s) {
     const int p = (int)(k & 1);
-    return esth_launch_mtgp(b->e->d_params, b->status[p], b->status[p ^ 1], b->streams, b->nstreams, b->R[p], 1, s);
+    return esth_launch_mtgp(b->e->d_params, b->status[p], b->status[p ^ 1], b->streams, b->nstreams, b->R[p], 1, s, 1, 0, 0,
+                            s == b->rng_stream);
 }
 
 static int capture_batch(esth_batch* b, int p) {

@@ -276,12 +276,18 @@ static int grid_for(uint64_t threads, int block) { return (int)((threads + block
 
 int esth_launch_mtgp(const uint32_t* d_params, const uint32_t* d_status_in, uint32_t* d_status_out,
                      const esth_mtgp_stream* d_streams, int nstreams, void* d_out, int float_mode, hipStream_t s,
-                     int nsteps, uint64_t out_step, uint64_t status_step) {
+                     int nsteps, uint64_t out_step, uint64_t status_step, bool beside) {
     if (nstreams <= 0 || nsteps <= 0) return ESTH_OK;
     if (nsteps > 1 && d_status_in == d_status_out)
         return esth_fail(ESTH_ERR_INVALID, "multi-step MTGP32 launch needs separate status buffers");
     const uint32_t mask = g_mtgp_table[3];
-    /* at most 8 resident work-groups per CU; more streams loop in the grid */
+    /* at most 8 resident work-groups per CU; more streams loop in the grid.
+     * 8 fill every wave slot and hold back what a step launches meanwhile (its
+     * frames' upload took 363 us instead of 52): beside a step's own launches,
+     * with 16 streams per CU and more, two (10,000 filters, 44,518 streams:
+     * 3.61 -> 3.52 ms per step; 2000 filters 0.707 -> 0.686 ms; at 1000
+     * filters, 4,600 streams, even; at 300 the words become the step's
+     * critical path, 148 -> 153 us) */
     static std::atomic<int> cus[64];
     int dev = 0;
     ESTH_HIP(hipGetDevice(&dev));
@@ -290,7 +296,8 @@ int esth_launch_mtgp(const uint32_t* d_params, const uint32_t* d_status_in, uint
         ESTH_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
         if (dev >= 0 && dev < 64) cus[dev].store(ncu, std::memory_order_relaxed);
     }
-    const int grid = std::min(nstreams, 8 * std::max(ncu, 1));
+    const int per_cu = beside && nstreams >= 16 * ncu ? 2 : 8;
+    const int grid = std::min(nstreams, per_cu * std::max(ncu, 1));
     hipLaunchKernelGGL(k_mtgp, dim3(grid), dim3(ESTH_MTGP_THREADS), 0, s, d_params, mask, d_status_in, d_status_out,
                        d_streams, (uint32_t)nstreams, (uint32_t*)d_out, float_mode, nsteps, out_step, status_step);
     ESTH_HIP(hipGetLastError());

@@ -56,10 +56,12 @@ int esth_check_desc(const esth_filter_desc* d, int* S, int* V);
 int esth_params_size(int model, size_t* sz);
 const uint32_t* esth_param_table();
 
-/* launchers shared by filters, batches and stage entry points */
+/* launchers shared by filters, batches and stage entry points.  beside: the
+ * words are generated beside a step's own launches, which should keep most of
+ * the chip */
 int esth_launch_mtgp(const uint32_t* d_params, const uint32_t* d_status_in, uint32_t* d_status_out,
                      const esth_mtgp_stream* d_streams, int nstreams, void* d_out, int float_mode, hipStream_t s,
-                     int nsteps = 1, uint64_t out_step = 0, uint64_t status_step = 0);
+                     int nsteps = 1, uint64_t out_step = 0, uint64_t status_step = 0, bool beside = false);
 /* frame: the step's frame in device memory; host_frame (non-null): the
  * frame passed by value as a kernel argument instead (frame unused) */
 int esth_launch_sample_weight(int model, float* state, uint32_t N, const float* R, const float* frame,
