@@ -568,10 +568,14 @@ int esth_launch_step_x(int model, uint32_t m, float* tmp, float* w, const float*
 }
 
 int esth_launch_argmax(int S, const float2* winner, uint32_t G, int log_w, const float* part, const float* sorted,
-                       uint32_t N, uint32_t m, float2* result, double* est, hipStream_t s) {
+                       uint32_t N, uint32_t m, float2* result, double* est, bool publish, hipStream_t s) {
     ESTH_TRY(esth_with_state_dim(S, [&](auto sv) {
-        hipLaunchKernelGGL(k_argmax<decltype(sv)::value>, dim3(1), dim3(1024), 0, s, winner, G, log_w, part, sorted, N, m,
-                           result, est);
+        if (publish)
+            hipLaunchKernelGGL((k_argmax<decltype(sv)::value, true>), dim3(1), dim3(1024), 0, s, winner, G, log_w, part,
+                               sorted, N, m, result, est);
+        else
+            hipLaunchKernelGGL((k_argmax<decltype(sv)::value, false>), dim3(1), dim3(1024), 0, s, winner, G, log_w, part,
+                               sorted, N, m, result, est);
         return ESTH_OK;
     }));
     ESTH_HIP(hipGetLastError());
@@ -904,7 +908,7 @@ extern "C" int esth_stage_argmax(const float* d_winner, uint32_t G, int weights,
     ESTH_HIP(hipMemset(part, 0, sizeof(float) * (size_t)G * 3));
     ESTH_HIP(hipMalloc((void**)&est, sizeof(double) * 8));
     int rc = esth_launch_argmax(1, (const float2*)d_winner, G, weights == ESTH_WEIGHTS_LOG, part, nullptr, 0, 1,
-                                (float2*)d_result, est, 0);
+                                (float2*)d_result, est, false, 0);
     ESTH_HIP(hipDeviceSynchronize());
     hipFree(part);
     hipFree(est);

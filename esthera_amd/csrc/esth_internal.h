@@ -130,9 +130,11 @@ int esth_launch_sample_sort(int model, uint32_t m, float* state, uint32_t N, uin
                             const float* host_frame = nullptr, const esth_mtgp_inline* mtgp = nullptr);
 /* whether esth_launch_sample_sort can carry MTGP32 work-groups at this m */
 bool esth_sample_sort_inline_rng(uint32_t m);
+/* publish: result is followed by the argmaxes' count, est as long as
+ * ESTH_EST_DOUBLES (esth_argmax_block, PUB) */
 int esth_launch_argmax(int S, const float2* winner, uint32_t G, int log_w, const float* part,
                        const float* sorted, uint32_t N, uint32_t m, float2* result, double* est,
-                       hipStream_t s);
+                       bool publish, hipStream_t s);
 int esth_launch_exchange(float* st, float* w, int S, uint32_t N, uint32_t m, uint32_t G, uint32_t t,
                          int topo, int dimx, int dimy, const float* bt_w, const float* bt_s,
                          uint32_t* top, hipStream_t s);

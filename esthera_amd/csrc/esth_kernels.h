@@ -40,13 +40,6 @@ __device__ __forceinline__ int esth_shfl_xor_i(int v, int mask) {
 __device__ __forceinline__ float esth_shfl_idx(float v, int src_lane) {
     return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(src_lane << 2, __builtin_bit_cast(int, v)));
 }
-__device__ __forceinline__ double esth_shfl_xor_d(double v, int mask) {
-    uint64_t u = __builtin_bit_cast(uint64_t, v);
-    int lo = esth_shfl_xor_i((int)(uint32_t)u, mask);
-    int hi = esth_shfl_xor_i((int)(uint32_t)(u >> 32), mask);
-    return __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-
 /* the halves of a 32- or 16-lane xor exchange (MASK 32 or 16), from one
  * v_permlane32_swap / v_permlane16_swap of v with itself: lo[i] is the value
  * of the lane of the pair {i, i ^ MASK} whose MASK bit is 0, hi[i] that of the
@@ -89,6 +82,17 @@ __device__ __forceinline__ int esth_xor_lane(int v) {
 template <int MASK>
 __device__ __forceinline__ float esth_xor_lane_f(float v) {
     return __builtin_bit_cast(float, esth_xor_lane<MASK>(__builtin_bit_cast(int, v)));
+}
+/* a wave's sum, pairing lanes K, K/2, ... 1 apart */
+template <int K>
+__device__ __forceinline__ double esth_bfly_sum_d(double v) {
+    if constexpr (K > 0) {
+        const uint64_t b = __builtin_bit_cast(uint64_t, v);
+        const uint32_t lo = (uint32_t)esth_xor_lane<K>((int)(uint32_t)b), hi = (uint32_t)esth_xor_lane<K>((int)(b >> 32));
+        return esth_bfly_sum_d<K / 2>(v + __builtin_bit_cast(double, (uint64_t)hi << 32 | lo));
+    } else {
+        return v;
+    }
 }
 /* butterfly sum over lane groups of size 2^LOG (fixed pairing order) */
 template <int K, int LIM>
@@ -844,18 +848,50 @@ __device__ __forceinline__ void esth_sort_keys(float (&key)[(esth_tile<LOGM, LAN
  * strided elements in order, loading them 16 at a time so the loads overlap.
  * The whole group then combines the sub-filters' posterior partial sums in
  * double and copies the best particle (rank 0 of the winning sub-filter,
- * read before any exchange).
+ * read before any exchange).  One work-group, so latency is all it costs, and
+ * a step whose estimate is read waits for it: loads that depend on nothing go
+ * out together, the best particle's beside the sums, and the wave sums go
+ * through DPP and lane swaps (4096 sub-filters read after every step: 132 ->
+ * 128 us a step).
  * est (doubles): [0] max log-weight, [1] sum w, [2..2+S) sum w x, [2+S] best w,
- * [3+S] best g, [4+S..4+2S) best particle. */
-template <int S, int NT>
+ * [3+S] best g, [4+S..4+2S) best particle.  PUB (single filters): est lies in
+ * coherent host memory and result is followed by the count of argmaxes run.
+ * One wave writes est past the caches (system scope), waits until its stores
+ * have arrived and then stores the count, one higher, to est[ESTH_EST_COUNT]:
+ * the host reads the estimate while the launch's other work-groups still
+ * resample.  (A system-scope release fence in that place writes the whole L2
+ * back beside them: dh6 512 x 2048 18.1 -> 19.2 ms per 200 steps.) */
+template <int S, int NT, bool PUB = false>
 __device__ __forceinline__ void esth_argmax_block(const float2* __restrict__ winner, uint32_t G, int log_w,
                                                   const float* __restrict__ part,
                                                   const float* __restrict__ best_src, size_t plane_stride,
                                                   uint32_t g_stride, float2* __restrict__ result,
                                                   double* __restrict__ est, float2* sc, float* smax, double* sd) {
     constexpr int NW = NT / 64;
+    constexpr int PM = 8;                       /* sub-filters per work-item whose maxima are loaded at once */
+    constexpr int U = (2 + S) <= 5 ? 4 : 2;     /* ... whose sums are */
     const int l = threadIdx.x;
     const int lane = l & 63, wid = l >> 6;
+    uint64_t count = 0;
+    if (PUB && l == 0) count = *reinterpret_cast<const uint64_t*>(result + 1) + 1;
+    /* every load that waits for nothing goes out first: maxima, winners, the
+     * first sums */
+    float pm[PM];
+    if (log_w) {
+#pragma unroll
+        for (int j = 0; j < PM; ++j) {
+            const uint32_t gi = (uint32_t)(l + j * NT);
+            pm[j] = gi < G ? part[(size_t)gi * (2 + S)] : -INFINITY;
+        }
+    }
+    auto fetch = [&](uint32_t g0, float (&q)[U][2 + S]) {
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const uint32_t gi = g0 + (uint32_t)(j * NT);
+#pragma unroll
+            for (int c = 0; c < 2 + S; ++c) q[j][c] = gi < G ? part[(size_t)gi * (2 + S) + c] : 0.0f;
+        }
+    };
     if (l < 128) {
         float2 acc = make_float2(log_w ? -INFINITY : -1.0f, -1.0f);
         for (uint32_t g0 = (uint32_t)l; g0 < G; g0 += 128u * 16u) {
@@ -871,22 +907,27 @@ __device__ __forceinline__ void esth_argmax_block(const float2* __restrict__ win
         }
         sc[l] = acc;
     }
-    float bmax = -INFINITY;
-    if (log_w) {   /* 8 loads in flight per work-item */
-        for (uint32_t g0 = (uint32_t)l; g0 < G; g0 += 8u * (uint32_t)NT) {
-            float pm[8];
+    float pg[U][2 + S];
+    fetch((uint32_t)l, pg);
+    if (log_w) {
+        float bmax = -INFINITY;
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < PM; ++j) bmax = pm[j] > bmax ? pm[j] : bmax;
+        for (uint32_t g0 = (uint32_t)(l + PM * NT); g0 < G; g0 += (uint32_t)(PM * NT)) {
+#pragma unroll
+            for (int j = 0; j < PM; ++j) {
                 const uint32_t gi = g0 + (uint32_t)(j * NT);
                 pm[j] = gi < G ? part[(size_t)gi * (2 + S)] : -INFINITY;
             }
 #pragma unroll
-            for (int j = 0; j < 8; ++j) bmax = pm[j] > bmax ? pm[j] : bmax;
+            for (int j = 0; j < PM; ++j) bmax = pm[j] > bmax ? pm[j] : bmax;
         }
         bmax = esth_bfly_max<1, 64>(bmax);
         if (lane == 0) smax[wid] = bmax;
     }
     __syncthreads();
+    float best = 0.0f;
+    bool have_best = false;
     if (l < 64) {   /* the reference tree over the 128 strided results */
         for (int off = 64; off > 0; off >>= 1) {
             if (l < off) {
@@ -896,6 +937,11 @@ __device__ __forceinline__ void esth_argmax_block(const float2* __restrict__ win
             }
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+        }
+        if (best_src && l < S) {   /* rank 0 of the winning sub-filter, component l */
+            const int gb = (int)sc[0].y;
+            have_best = gb >= 0 && (uint32_t)gb < G;
+            if (have_best) best = best_src[(size_t)l * plane_stride + (size_t)gb * g_stride];
         }
     }
     float gmax = 0.0f;
@@ -908,15 +954,8 @@ __device__ __forceinline__ void esth_argmax_block(const float2* __restrict__ win
 #pragma unroll
     for (int c = 0; c < 2 + S; ++c) a[c] = 0.0;
     /* the same per-work-item order of sub-filters, U of them loaded at once */
-    constexpr int U = (2 + S) <= 5 ? 4 : 2;
     for (uint32_t g0 = (uint32_t)l; g0 < G; g0 += (uint32_t)U * (uint32_t)NT) {
-        float pg[U][2 + S];
-#pragma unroll
-        for (int j = 0; j < U; ++j) {
-            const uint32_t gi = g0 + (uint32_t)(j * NT);
-#pragma unroll
-            for (int c = 0; c < 2 + S; ++c) pg[j][c] = gi < G ? part[(size_t)gi * (2 + S) + c] : 0.0f;
-        }
+        if (g0 != (uint32_t)l) fetch(g0, pg);
 #pragma unroll
         for (int j = 0; j < U; ++j) {
             if (g0 + (uint32_t)(j * NT) >= G) break;
@@ -927,30 +966,40 @@ __device__ __forceinline__ void esth_argmax_block(const float2* __restrict__ win
     }
 #pragma unroll
     for (int c = 1; c < 2 + S; ++c) {
-        double v = a[c];
-        for (int k = 32; k > 0; k >>= 1) v += esth_shfl_xor_d(v, k);
+        const double v = esth_bfly_sum_d<32>(a[c]);
         if (lane == 0) sd[wid * (2 + S) + c] = v;
     }
     __syncthreads();
+    auto put = [&](int i, double v) {
+        if constexpr (PUB) __hip_atomic_store(est + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        else est[i] = v;
+    };
     if (l == 0) {
         result[0] = sc[0];
-        est[0] = (double)gmax;
+        put(0, (double)gmax);
 #pragma unroll
         for (int c = 1; c < 2 + S; ++c) {
             double v = 0.0;
             for (int i = 0; i < NW; ++i) v += sd[i * (2 + S) + c];
-            est[c] = v;
+            put(c, v);
         }
-        est[2 + S] = (double)sc[0].x;
-        est[3 + S] = (double)sc[0].y;
+        put(2 + S, (double)sc[0].x);
+        put(3 + S, (double)sc[0].y);
     }
-    if (best_src && l < S) {   /* rank 0 of the winning sub-filter, component l */
-        int gb = (int)sc[0].y;
-        if (gb >= 0 && (uint32_t)gb < G) est[4 + S + l] = (double)best_src[(size_t)l * plane_stride + (size_t)gb * g_stride];
+    if (have_best) put(4 + S + l, (double)best);
+    if constexpr (PUB) {
+        if (l < ESTH_WAVE) {   /* the wave that wrote est */
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            if (l == 0) {
+                *reinterpret_cast<uint64_t*>(result + 1) = count;
+                __hip_atomic_store(reinterpret_cast<uint64_t*>(est + ESTH_EST_COUNT), count, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
     }
 }
 
-template <int S>
+template <int S, bool PUB>
 __global__ __launch_bounds__(1024) void k_argmax(const float2* __restrict__ winner, uint32_t G,
                                                  int log_w, const float* __restrict__ part,
                                                  const float* __restrict__ sorted, uint32_t N,
@@ -959,7 +1008,7 @@ __global__ __launch_bounds__(1024) void k_argmax(const float2* __restrict__ winn
     __shared__ float2 sc[128];
     __shared__ float smax[16];
     __shared__ double sd[16 * (2 + S)];
-    esth_argmax_block<S, 1024>(winner, G, log_w, part, sorted, N, m, result, est, sc, smax, sd);
+    esth_argmax_block<S, 1024, PUB>(winner, G, log_w, part, sorted, N, m, result, est, sc, smax, sd);
 }
 
 /* Sorted weights in place, gathered state to `sorted`, winner (w[0], g),
@@ -1709,7 +1758,7 @@ __global__ __launch_bounds__(256) void k_resample_argmax(float* __restrict__ st_
     if (mi.n && esth_mtgp_inline_wg(mi, mst)) return;
     const uint32_t bx = blockIdx.x - (uint32_t)mi.n;
     if (bx == 0) {
-        esth_argmax_block<S, 256>(winner, G, log_w, part, best_src, plane_stride, g_stride, result, est, sc, smax, sd);
+        esth_argmax_block<S, 256, true>(winner, G, log_w, part, best_src, plane_stride, g_stride, result, est, sc, smax, sd);
         return;
     }
     const int lane = threadIdx.x & (ESTH_WAVE - 1);
@@ -1913,7 +1962,7 @@ __global__ __launch_bounds__(256) void k_resample2_argmax(float* __restrict__ st
     if (mi.n && esth_mtgp_inline_wg(mi, reinterpret_cast<uint32_t*>(cdf_s))) return;
     const uint32_t bx = blockIdx.x - (uint32_t)mi.n;
     if (bx == 0) {
-        esth_argmax_block<S, 256>(winner, G, log_w, part, best_src, plane_stride, g_stride, result, est, sc, smax, sd);
+        esth_argmax_block<S, 256, true>(winner, G, log_w, part, best_src, plane_stride, g_stride, result, est, sc, smax, sd);
         return;
     }
     const int wv = (int)esth_block_wave();   /* 0..3: sub-filter wv / 2, half wv % 2 */
@@ -1963,7 +2012,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     if (mi.n && esth_mtgp_inline_wg(mi, reinterpret_cast<uint32_t*>(lds))) return;
     const uint32_t b0 = (uint32_t)mi.n;
     if (blockIdx.x == b0) {
-        esth_argmax_block<S, 256>(winner_k, G, log_w, part_k, best_k, (size_t)G * xk.t, xk.t, result, est, sc, smax,
+        esth_argmax_block<S, 256, true>(winner_k, G, log_w, part_k, best_k, (size_t)G * xk.t, xk.t, result, est, sc, smax,
                                   sd);
         return;
     }
@@ -2538,7 +2587,7 @@ __global__ __launch_bounds__(256) void k_alias_argmax_w(float* __restrict__ st_m
     }
     const uint32_t bx = blockIdx.x - (uint32_t)mi.n;
     if (bx == 0) {
-        esth_argmax_block<S, WPB * ESTH_WAVE>(winner, G, log_w, part, best_src, plane_stride, g_stride, result, est, sc,
+        esth_argmax_block<S, WPB * ESTH_WAVE, true>(winner, G, log_w, part, best_src, plane_stride, g_stride, result, est, sc,
                                               smax, sd);
         return;
     }

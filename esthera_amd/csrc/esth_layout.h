@@ -111,4 +111,9 @@ static inline void esth_torus_dims(uint32_t G, int* dimx, int* dimy) {
     *dimy = (int)(G / x);
 }
 
+/* a filter's posterior sums and best particle, then the count of argmaxes
+ * that have written them */
+#define ESTH_EST_COUNT (4 + 2 * ESTH_MAX_STATE_DIM)
+#define ESTH_EST_DOUBLES (ESTH_EST_COUNT + 1)
+
 #endif /* ESTH_LAYOUT_H */
