@@ -274,6 +274,19 @@ void esth_engine_release(esth_engine* e, void* p, size_t bytes) {
 /* ============================================================ launchers */
 static int grid_for(uint64_t threads, int block) { return (int)((threads + block - 1) / block); }
 
+/* compute units of the current device */
+static int esth_cus() {
+    static std::atomic<int> cus[64];
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    n = cus[dev].load(std::memory_order_relaxed);
+    if (n <= 0) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+        cus[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
+}
+
 int esth_launch_mtgp(const uint32_t* d_params, const uint32_t* d_status_in, uint32_t* d_status_out,
                      const esth_mtgp_stream* d_streams, int nstreams, void* d_out, int float_mode, hipStream_t s,
                      int nsteps, uint64_t out_step, uint64_t status_step, bool beside) {
@@ -288,16 +301,9 @@ int esth_launch_mtgp(const uint32_t* d_params, const uint32_t* d_status_in, uint
      * 3.61 -> 3.52 ms per step; 2000 filters 0.707 -> 0.686 ms; at 1000
      * filters, 4,600 streams, even; at 300 the words become the step's
      * critical path, 148 -> 153 us) */
-    static std::atomic<int> cus[64];
-    int dev = 0;
-    ESTH_HIP(hipGetDevice(&dev));
-    int ncu = (dev >= 0 && dev < 64) ? cus[dev].load(std::memory_order_relaxed) : 0;
-    if (ncu <= 0) {
-        ESTH_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-        if (dev >= 0 && dev < 64) cus[dev].store(ncu, std::memory_order_relaxed);
-    }
+    const int ncu = esth_cus();
     const int per_cu = beside && nstreams >= 16 * ncu ? 2 : 8;
-    const int grid = std::min(nstreams, per_cu * std::max(ncu, 1));
+    const int grid = std::min(nstreams, per_cu * ncu);
     hipLaunchKernelGGL(k_mtgp, dim3(grid), dim3(ESTH_MTGP_THREADS), 0, s, d_params, mask, d_status_in, d_status_out,
                        d_streams, (uint32_t)nstreams, (uint32_t*)d_out, float_mode, nsteps, out_step, status_step);
     ESTH_HIP(hipGetLastError());
@@ -663,11 +669,27 @@ static void launch_resample_argmax_t(float* st_main, const float* st_tmp, const 
                                      const esth_mtgp_inline& mi, hipStream_t s) {
     /* two waves per sub-filter for m >= 512 where the work-group's two
      * sub-filters' CDFs and staged planes fit in 48 KB of LDS (at m = 256 in
-     * the batched classes the halves were too short to pay for the barriers) */
-    if constexpr (LOGM >= 9 && (1 + S) * (1 << LOGM) <= 6144) {
-        hipLaunchKernelGGL((k_resample2_argmax<LOGM, S>), dim3(mi.n + 1 + (G + 1) / 2), dim3(256), 0, s, st_main, st_tmp, w,
-                           rnd, N, G, thr, systematic, log_w, winner, part, best_src, plane_stride, g_stride, result,
-                           est, xch, carry, layout, mi);
+     * the batched classes the halves were too short to pay for the barriers).
+     * Where they do not fit, four waves while the sub-filters are few: one
+     * wave each is then a long chain on a chip mostly idle (robotarm5 at m =
+     * 1024, whole steps, one wave against four: 8 sub-filters 34.6 and 25.3
+     * us, 500 52.2 and 43.6 (the launch 28 and 16), 768 60.1 and 58.6, 1024
+     * 117.1 and 118.7; dh6 at 512: 8 22.3 and 18.6, 256 28.6 and 26.5, 500
+     * 35.2 and 38.4; at 1024: 512 72.5 and 68.0).  For the smaller ones the
+     * wave counts are even or worse (unicycle and robotarm5 at m = 256 with
+     * two waves 0-5 % slower, at 512 with four -1 to +4 %). */
+    constexpr bool halves = LOGM >= 9 && (1 + S) * (1 << LOGM) <= 6144;
+    auto launch2 = [&](auto waves) {
+        constexpr int W = decltype(waves)::value;
+        hipLaunchKernelGGL((k_resample2_argmax<LOGM, S, W>), dim3(mi.n + 1 + (G + 4 / W - 1) / (4 / W)), dim3(256), 0, s,
+                           st_main, st_tmp, w, rnd, N, G, thr, systematic, log_w, winner, part, best_src, plane_stride,
+                           g_stride, result, est, xch, carry, layout, mi);
+    };
+    if constexpr (LOGM >= 9 && !halves) {
+        if (G <= (uint32_t)((LOGM >= 10 ? 3 : 1) * esth_cus())) return launch2(std::integral_constant<int, 4>{});
+    }
+    if constexpr (halves) {
+        launch2(std::integral_constant<int, 2>{});
     } else {
         using TL = esth_tile<LOGM>;
         const uint64_t waves = (G + (ESTH_WAVE / TL::LPS) - 1) / (ESTH_WAVE / TL::LPS);

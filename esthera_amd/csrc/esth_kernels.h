@@ -1938,9 +1938,12 @@ __device__ __forceinline__ void esth_resample_sub2(float* __restrict__ st_main, 
     }
 }
 
-/* k_resample_argmax with two waves per sub-filter (m >= 256): work-group 0
- * the argmax, each other work-group of four waves two sub-filters */
-template <int LOGM, int S>
+/* k_resample_argmax with W = 2 or 4 waves per sub-filter (m >= 512):
+ * work-group 0 the argmax, each other work-group of four waves 4 / W
+ * sub-filters.  With four waves a lane holds m / 256 particles of every plane
+ * instead of m / 64: 73 registers for nine planes at m = 1024 instead of 188,
+ * and a chain a third as long (500 sub-filters 28 -> 16 us; bytes alone 8) */
+template <int LOGM, int S, int W>
 __global__ __launch_bounds__(256) void k_resample2_argmax(float* __restrict__ st_main,
                                                           const float* __restrict__ st_tmp, const float* w,
                                                           const float* __restrict__ rnd, uint32_t N, uint32_t G,
@@ -1952,26 +1955,26 @@ __global__ __launch_bounds__(256) void k_resample2_argmax(float* __restrict__ st
                                                           double* __restrict__ est, esth_xch xch, int carry,
                                                           int layout, const esth_mtgp_inline mi) {
     constexpr int M = 1 << LOGM;
-    __shared__ __align__(16) float cdf_s[2][M];
-    __shared__ __align__(16) float stage_s[2][S * M];
-    __shared__ float xl_s[2][4];
+    __shared__ __align__(16) float cdf_s[4 / W][M];
+    __shared__ __align__(16) float stage_s[4 / W][S * M];
+    __shared__ float xl_s[4 / W][2 * W];
     __shared__ float2 sc[128];
     __shared__ float smax[4];
     __shared__ double sd[4 * (2 + S)];
-    static_assert(2 * M >= ESTH_MTGP_LDS, "an MTGP32 ring fits where the prefix sums go");
-    if (mi.n && esth_mtgp_inline_wg(mi, reinterpret_cast<uint32_t*>(cdf_s))) return;
+    static_assert((4 / W) * S * M >= ESTH_MTGP_LDS, "an MTGP32 ring fits where the planes go");
+    if (mi.n && esth_mtgp_inline_wg(mi, reinterpret_cast<uint32_t*>(stage_s))) return;
     const uint32_t bx = blockIdx.x - (uint32_t)mi.n;
     if (bx == 0) {
         esth_argmax_block<S, 256, true>(winner, G, log_w, part, best_src, plane_stride, g_stride, result, est, sc, smax, sd);
         return;
     }
-    const int wv = (int)esth_block_wave();   /* 0..3: sub-filter wv / 2, half wv % 2 */
-    const int j = wv >> 1;
-    uint32_t g = (bx - 1) * 2u + (uint32_t)j;
+    const int wv = (int)esth_block_wave();   /* 0..3: sub-filter wv / W, part wv % W */
+    const int j = wv / W;
+    uint32_t g = (bx - 1) * (4u / W) + (uint32_t)j;
     const bool valid = g < G;
     if (!valid) g = G - 1;
-    esth_resample_sub2<LOGM, S>(st_main, st_tmp, w, rnd, N, g, valid, thr, systematic, log_w, cdf_s[j], stage_s[j],
-                                xl_s[j], wv & 1, xch, carry, const_cast<float*>(w), layout);
+    esth_resample_sub2<LOGM, S, false, W>(st_main, st_tmp, w, rnd, N, g, valid, thr, systematic, log_w, cdf_s[j], stage_s[j],
+                                xl_s[j], wv % W, xch, carry, const_cast<float*>(w), layout);
 }
 
 /* One launch per step across the step boundary: work-group b resamples
