@@ -209,6 +209,7 @@ static void filter_free(esth_filter* f) {
     if (!f) return;
     hipSetDevice(f->e->device);
     if (f->stream) hipStreamSynchronize(f->stream);
+    if (f->rng_stream) hipStreamSynchronize(f->rng_stream);   /* the next block may still be written */
     for (int i = 0; i < ESTH_FRAME_RING; ++i)
         if (f->gexec[i]) hipGraphExecDestroy(f->gexec[i]);
     for (auto& a : f->allocs) esth_engine_release(f->e, a.first, a.second);
