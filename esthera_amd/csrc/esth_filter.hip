@@ -87,6 +87,7 @@ struct esth_filter {
      * us, 256,000 with the alias resampler 52.6 -> 40.9, 2M 136 -> 128) */
     double* est = nullptr;
     uint64_t argmaxes = 0;   /* launches with an argmax enqueued so far */
+    bool recount = false;    /* ... give or take one that failed and may have run */
     /* the cross-step launch (k_step_x): step n's resampling runs at the start
      * of step n + 1's launch.  Sorted-side buffers alternate by step parity
      * (winner/part/bt_w/bt_s for even steps, *2 for odd ones) and the words
@@ -662,13 +663,22 @@ static int enqueue_cross(esth_filter* f, uint64_t n, const float* d_frame, const
     return ESTH_OK;
 }
 
+/* rc of enqueuing a launch with an argmax: it is counted once it is known to
+ * run.  A failed one may have run all the same (an error left by an earlier
+ * call is reported by the next launch): the next estimate takes the count
+ * from the device. */
+static int counted(esth_filter* f, int rc) {
+    if (rc == ESTH_OK) f->argmaxes++;
+    else f->recount = true;
+    return rc;
+}
+
 /* run the resampling the last step left pending */
 static int flush(esth_filter* f) {
     if (!f->pending) return ESTH_OK;
     ESTH_HIP(hipSetDevice(f->e->device));
     f->pending = false;
-    f->argmaxes++;
-    return enqueue_resample(f, f->steps - 1, nullptr);
+    return counted(f, enqueue_resample(f, f->steps - 1, nullptr));
 }
 
 /* Capture the kernels of a step that reads word block parity p, position kk
@@ -752,20 +762,19 @@ extern "C" int esth_filter_step(esth_filter* f, const void* control, const void*
         ESTH_HIP(hipMemcpyAsync(dfr, hf, sizeof(float) * ESTH_FRAME_FLOATS, hipMemcpyHostToDevice, f->stream));
         ESTH_HIP(hipEventRecord(f->frame_ev[slot], f->stream));
         f->frame_used[slot] = true;
-        if (mode != ESTH_GRAPH_SAMPLE) f->argmaxes++;
-        ESTH_HIP(hipGraphLaunch(f->gexec[slot], f->stream));
+        const hipError_t err = hipGraphLaunch(f->gexec[slot], f->stream);
+        const int rc = err == hipSuccess ? ESTH_OK : esth_fail(ESTH_ERR_DEVICE, "graph launch: %s", hipGetErrorString(err));
+        ESTH_TRY(mode != ESTH_GRAPH_SAMPLE ? counted(f, rc) : rc);
         if (cross) f->pending = true;
     } else if (cross) {
         if (f->pending) {
-            f->argmaxes++;
-            ESTH_TRY(enqueue_cross(f, n, nullptr, hf, ev, &work));
+            ESTH_TRY(counted(f, enqueue_cross(f, n, nullptr, hf, ev, &work)));
         } else {
             ESTH_TRY(enqueue_sample(f, n, nullptr, hf, ev, &work));
         }
         f->pending = true;
     } else {
-        f->argmaxes++;
-        ESTH_TRY(enqueue_step(f, n, nullptr, hf, ev, &work));
+        ESTH_TRY(counted(f, enqueue_step(f, n, nullptr, hf, ev, &work)));
     }
     ESTH_TRY(rng_after_step(f, in));
     f->steps++;
@@ -894,21 +903,23 @@ extern "C" int esth_filter_stage_times(esth_filter* f, float us[6]) {
 }
 
 /* until the last argmax enqueued has published its estimate: its count,
- * polled for up to ESTH_POLL_US, beyond that (long queues, a launch that
- * failed) the stream's end */
+ * polled for up to ESTH_POLL_US, beyond that (long queues) the stream's end */
 static int wait_estimate(esth_filter* f) {
     const std::atomic<uint64_t>* count = reinterpret_cast<const std::atomic<uint64_t>*>(f->est + ESTH_EST_COUNT);
     const auto t0 = std::chrono::steady_clock::now();
-    for (int i = 1; count->load(std::memory_order_acquire) < f->argmaxes; ++i) {
-        if (i % 64 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(ESTH_POLL_US)) {
-            ESTH_HIP(hipStreamSynchronize(f->stream));
-            return ESTH_OK;
-        }
+    for (int i = 1; !f->recount; ++i) {
+        if (count->load(std::memory_order_acquire) >= f->argmaxes) return ESTH_OK;
+        if (i % 64 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(ESTH_POLL_US)) break;
 #if !defined(__HIP_DEVICE_COMPILE__)
         __builtin_ia32_pause();
 #endif
     }
-    return ESTH_OK;
+    ESTH_HIP(hipStreamSynchronize(f->stream));
+    const uint64_t done = count->load(std::memory_order_acquire);
+    const bool lost = !f->recount && done < f->argmaxes;
+    f->argmaxes = done;
+    f->recount = false;
+    return lost ? esth_fail(ESTH_ERR_DEVICE, "the step's estimate was not written") : ESTH_OK;
 }
 
 extern "C" int esth_filter_estimate(esth_filter* f, esth_estimate* out) {

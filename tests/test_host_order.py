@@ -1,0 +1,109 @@
+"""The order in which filters and batches enqueue their work, and what they do
+when a call to the runtime fails, on the CPU: libesthera.so runs on a stand-in
+for the HIP runtime (fake_hip.cpp) that launches nothing and logs every call.
+Each scenario runs in a process of its own, where the stand-in is loaded first."""
+import ctypes as C
+import os
+import re
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+class Fake:
+    """The stand-in: its log, and failures asked for by a part of a log line."""
+
+    def __init__(self, path):
+        self.lib = C.CDLL(path, mode=C.RTLD_GLOBAL)
+        self.lib.fake_log.restype = C.c_char_p
+        self.lib.fake_fail.argtypes = [C.c_char_p]
+
+    def log(self):
+        return self.lib.fake_log().decode().splitlines()
+
+    def take(self):
+        lines = self.log()
+        self.lib.fake_clear()
+        return lines
+
+    def fail(self, what):
+        self.lib.fake_fail(what.encode())
+
+
+def walk(ea, m=128, G=12, **k):
+    """A random walk's filter and its step's arguments."""
+    d = ea.filter_desc(ea.MODEL_RANDOMWALK3, m=m, G=G, weights=ea.WEIGHTS_LOG, resampler=ea.RESAMPLE_SYSTEMATIC, **k)
+    p, c, z, _ = ea.randomwalk3_scenario(3, 1)
+    return d, p, (c[0], z[0], 0.1)
+
+
+def fails(ea, call, *args):
+    try:
+        call(*args)
+    except ea.EsthError:
+        return True
+    return False
+
+
+def failed_argmax(ea, fake):
+    d, p, args = walk(ea)
+    fake.take()
+    f = ea.Filter(ea.Engine(0), d, p)
+    # the estimate's pinned buffer: 4 + 2 * 16 doubles and the count of argmaxes that have published one
+    at = [int(l.split()[1], 16) for l in fake.take() if l.startswith("hipHostMalloc") and l.endswith("bytes 296")]
+    count = C.c_uint64.from_address(at[0] + 288)
+    f.init_uniform([0.0, 0.0, 0.0])
+
+    def waits():
+        fake.take()
+        f.estimate()
+        return any(l.startswith("hipStreamSynchronize") for l in fake.take())
+
+    f.step(*args)
+    count.value = 1
+    assert not waits()
+    # a failed launch that did not run
+    fake.fail("k_resample_argmax")
+    assert fails(ea, f.step, *args)
+    assert waits(), "after a failed launch the estimate waits for the stream"
+    f.step(*args)
+    count.value = 2
+    assert not waits(), "the count is short for good"
+    # one that ran although the call failed
+    fake.fail("k_resample_argmax")
+    assert fails(ea, f.step, *args)
+    count.value = 3
+    assert waits()
+    f.step(*args)
+    assert fails(ea, f.estimate), "an estimate that was not published is no estimate"
+    f.step(*args)
+    count.value = 4
+    assert not waits()
+
+
+SCENARIOS = [failed_argmax]
+
+
+@pytest.fixture(scope="session")
+def stand_in(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.run(["g++", "-shared", "-fPIC", "-O1", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "fake_hip.cpp"), "-o", out], check=True)
+    return out
+
+
+@pytest.mark.parametrize("scenario", [s.__name__ for s in SCENARIOS])
+def test_host_order(scenario, stand_in):
+    r = subprocess.run([sys.executable, os.path.abspath(__file__), scenario, stand_in], capture_output=True, text=True,
+                       timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+if __name__ == "__main__":
+    fake = Fake(sys.argv[2])
+    sys.path.insert(0, os.path.dirname(HERE))
+    import esthera_amd
+    globals()[sys.argv[1]](esthera_amd, fake)
