@@ -242,7 +242,7 @@ struct esth_batch {
      * copy, after one wait for the steps enqueued so far (10,000 estimates
      * 140 -> 10 ms; the argmax launch 39 -> 47 us) */
     double* est = nullptr;
-    uint64_t waited = 0;   /* steps known to have run */
+    bool waited = true;   /* everything enqueued so far is known to have run */
     uint32_t* top = nullptr;
     std::vector<std::pair<void*, size_t>> allocs;
     /* host */
@@ -722,6 +722,7 @@ extern "C" int esth_batch_step(esth_batch* b, const void* controls, size_t contr
     /* RNG: this step's words (if not prefetched) and the next step's on the RNG stream */
     hipStream_t s = b->stream;
     const uint64_t n = b->steps;
+    b->waited = false;   /* also where a call below fails: kernels enqueued before it still run */
     bool forked = false;
     if (!b->rng_ready) {
         ESTH_TRY(launch_rng_b(b, n, s));
@@ -770,9 +771,9 @@ extern "C" int esth_batch_use_graph(esth_batch* b, int enable) {
 
 extern "C" int esth_batch_estimate(esth_batch* b, int i, esth_estimate* out) {
     if (!b || !out || i < 0 || i >= b->n) return esth_fail(ESTH_ERR_INVALID, "batch estimate: bad filter %d", i);
-    if (b->waited != b->steps) {
+    if (!b->waited) {
         ESTH_HIP(hipStreamSynchronize(b->stream));
-        b->waited = b->steps;
+        b->waited = true;
     }
     const int S = b->S;
     const double* h = b->est + (size_t)i * (4 + 2 * ESTH_MAX_STATE_DIM);

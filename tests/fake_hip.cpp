@@ -99,6 +99,18 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { *s = (hipStream_
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t s) { return say("hipStreamSynchronize stream %d", id(s)); }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t e, unsigned) { return say("hipStreamWaitEvent stream %d event %d", id(s), id(e)); }
+hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) { return say("hipStreamBeginCapture stream %d", id(s)); }
+hipError_t hipStreamEndCapture(hipStream_t s, hipGraph_t* g) {
+    *g = (hipGraph_t)++g_handles;
+    return say("hipStreamEndCapture stream %d", id(s));
+}
+hipError_t hipGraphInstantiate(hipGraphExec_t* x, hipGraph_t, hipGraphNode_t*, char*, size_t) {
+    *x = (hipGraphExec_t)++g_handles;
+    return hipSuccess;
+}
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t s) { return say("hipGraphLaunch stream %d", id(s)); }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned f) { *e = (hipEvent_t)++g_handles; return say("event %d flags %x", id(*e), f); }
 hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }

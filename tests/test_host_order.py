@@ -84,7 +84,27 @@ def failed_argmax(ea, fake):
     assert not waits()
 
 
-SCENARIOS = [failed_argmax]
+def failed_batch_step(ea, fake):
+    d, p, (c, z, dt) = walk(ea, rng=ea.RNG_MTGP_PER_FILTER)
+    b = ea.Batch(ea.Engine(0), [d, d], [p, p])
+    cs, zs, dts = (ea.RandomWalk3Control * 2)(c, c), (ea.RandomWalk3Measurement * 2)(z, z), [dt, dt]
+    fake.take()
+    b.step(cs, zs, dts)
+    last = fake.take()[-1]   # an event after the step's kernels
+    assert last.startswith("hipEventRecord")
+    b.step(cs, zs, dts)
+    b.estimate(0)
+    fake.take()
+    b.estimate(1)
+    assert not fake.take(), "one wait for all estimates of a step"
+    fake.fail(last)   # the third step, its kernels enqueued
+    assert fails(ea, b.step, cs, zs, dts)
+    assert any("GraphLaunch" in l for l in fake.take())
+    b.estimate(0)
+    assert any(l.startswith("hipStreamSynchronize") for l in fake.take()), "kernels may still write the estimates"
+
+
+SCENARIOS = [failed_argmax, failed_batch_step]
 
 
 @pytest.fixture(scope="session")
