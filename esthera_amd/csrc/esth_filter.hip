@@ -320,10 +320,6 @@ extern "C" int esth_filter_create(esth_engine* e, const esth_filter_desc* d, con
     if (err == hipSuccess) err = hipHostMalloc((void**)&f->est, est_bytes, hipHostMallocMapped | hipHostMallocCoherent);
     if (err != hipSuccess) { filter_free(f); return esth_fail(ESTH_ERR_DEVICE, "stream/pinned: %s", hipGetErrorString(err)); }
     memset(f->est, 0, est_bytes);
-    if (hipMemset(f->result, 0, sizeof(float2) + sizeof(uint64_t)) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
-        filter_free(f);
-        return esth_fail(ESTH_ERR_DEVICE, "argmax count");
-    }
     /* RNG status: make_kernel_data32 (mtgp32-opencl.c:31-60), stream j seeded seed + j + 1 */
     std::vector<uint32_t> st((size_t)ESTH_MTGP_N * f->K);
     std::vector<esth_mtgp_stream> sd(f->K);
@@ -334,6 +330,10 @@ extern "C" int esth_filter_create(esth_engine* e, const esth_filter_desc* d, con
     err = hipMemcpy(status_slot(f, 1, f->B), st.data(), st.size() * sizeof(uint32_t), hipMemcpyHostToDevice);
     if (err == hipSuccess) err = hipMemcpy(f->streams, sd.data(), sd.size() * sizeof(esth_mtgp_stream), hipMemcpyHostToDevice);
     if (err == hipSuccess) err = hipMemset(f->w, 0, sizeof(float) * f->N);
+    /* the argmaxes' count: there when the copy returns, as the rest; a wait for
+     * the device would stop at what other filters have queued */
+    const unsigned char none[sizeof(float2) + sizeof(uint64_t)] = {};
+    if (err == hipSuccess) err = hipMemcpy(f->result, none, sizeof(none), hipMemcpyHostToDevice);
     if (err != hipSuccess) { filter_free(f); return esth_fail(ESTH_ERR_DEVICE, "init upload: %s", hipGetErrorString(err)); }
     *out = f;
     return ESTH_OK;

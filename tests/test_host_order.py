@@ -104,7 +104,17 @@ def failed_batch_step(ea, fake):
     assert any(l.startswith("hipStreamSynchronize") for l in fake.take()), "kernels may still write the estimates"
 
 
-SCENARIOS = [failed_argmax, failed_batch_step]
+def creation_waits_for_no_stream(ea, fake):
+    d, p, _ = walk(ea)
+    e = ea.Engine(0)
+    fake.take()
+    f = ea.Filter(e, d, p)
+    log = fake.take()
+    assert f.h and sum(l.startswith("hipMemcpy") for l in log) >= 2   # statuses and streams go up
+    assert not [l for l in log if "Synchronize" in l]
+
+
+SCENARIOS = [failed_argmax, failed_batch_step, creation_waits_for_no_stream]
 
 
 @pytest.fixture(scope="session")
