@@ -257,14 +257,14 @@ extern "C" int esth_filter_create(esth_engine* e, const esth_filter_desc* d, con
     f->dimy = d->torus_dimy;
     if (d->topology == ESTH_TOPO_TORUS && (f->dimx <= 0 || f->dimy <= 0)) esth_torus_dims(f->G, &f->dimx, &f->dimy);
     for (int i = 0; i < ESTH_FRAME_RING; ++i) hipEventCreateWithFlags(&f->frame_ev[i], hipEventDisableTiming);
-    /* ESTH_RNG_BLOCK_STEPS (1..ESTH_RNG_BLOCK) overrides the block length */
+    /* ESTH_RNG_BLOCK_STEPS (1..ESTH_RNG_BLOCK): the second stream in blocks of that length (1: inline words stay) */
     f->inline_rng = (!f->fuse_sample_sort || esth_sample_sort_inline_rng(f->m)) && inline_rng_pays(f);
     uint64_t blk = 0;
     if (const char* ev = getenv("ESTH_RNG_BLOCK_STEPS")) {
         const long v = strtol(ev, nullptr, 10);
         if (v >= 1 && v <= ESTH_RNG_BLOCK) blk = (uint64_t)v;
     }
-    f->carried = !f->inline_rng && (blk == 0 || blk == ESTH_RNG_BLOCK_DEFAULT) && carried_rng_pays(f);
+    f->carried = !f->inline_rng && blk == 0 && carried_rng_pays(f);
     const uint64_t two = 2ull * sizeof(float) * f->words;   /* two blocks of one step */
     if (blk == 0)
         blk = f->inline_rng ? 1

@@ -114,7 +114,38 @@ def creation_waits_for_no_stream(ea, fake):
     assert not [l for l in log if "Synchronize" in l]
 
 
-SCENARIOS = [failed_argmax, failed_batch_step, creation_waits_for_no_stream]
+def steps_per_block(log):
+    """(stream, steps) of each generator launch."""
+    return [(l.split()[3], int(l.split()[5])) for l in log if "6k_mtgp" in l]
+
+
+def carried_words(ea, fake):
+    """Small filters' words ride in the step's own launches (those of test_gpu_carried_words among them): the
+    generator is launched ahead of the first step only.  A block length asked for puts any filter's words on the
+    second stream, in blocks of that length."""
+    e = ea.Engine(0)
+    for m, G, L, res in ((256, 64, 4, ea.RESAMPLE_SYSTEMATIC), (64, 100, 4, ea.RESAMPLE_ALIAS),
+                         (512, 512, 20, ea.RESAMPLE_ALIAS)):
+        p, c, z, _ = ea.unicycle_scenario(3, L, 20.0, 1)
+        d = ea.filter_desc(ea.MODEL_UNICYCLE, m=m, G=G, t=1, resampler=res, weights=ea.WEIGHTS_LOG, seed=77)
+        for block in (0, 1, 2, 3, 4):
+            os.environ.pop("ESTH_RNG_BLOCK_STEPS", None)
+            if block:
+                os.environ["ESTH_RNG_BLOCK_STEPS"] = str(block)
+            f = ea.Filter(e, d, p)
+            f.init_uniform([0.0, 0.0, 0.0])
+            fake.take()
+            for _ in range(8):
+                f.step(c[0], z[0], 0.1)
+            got = steps_per_block(fake.take())
+            if block == 0:
+                assert len(got) == 1 and got[0][1] == 1, (m, G, got)
+            else:
+                assert f.rng_mode() == (False, block)
+                assert len({s for s, _ in got}) == 2 and got[-1][1] == block, (m, G, block, got)
+
+
+SCENARIOS = [failed_argmax, failed_batch_step, creation_waits_for_no_stream, carried_words]
 
 
 @pytest.fixture(scope="session")
