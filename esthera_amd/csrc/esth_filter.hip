@@ -32,8 +32,7 @@
  * (134 MB) 9.13, 9.05, 8.93 ms; dh6 512 x 2048 (235 MB) 18.56, 18.21, 18.46;
  * unicycle 512 x 4096 (268 MB) 14.54, 14.33, 14.93: the words of two blocks
  * have to lie in the 256 MB Infinity Cache with what the step's launches
- * read.  Blocks of 8 gain 1-3 % more at 128 x 3001, but a run's first step
- * waits for a whole block. */
+ * read.  Blocks of 8 gain 1-3 % more at 128 x 3001 for twice the memory. */
 #define ESTH_RNG_BLOCK 8
 #define ESTH_RNG_BLOCK_DEFAULT 2
 #define ESTH_RNG_BLOCK_LONG 4
@@ -69,7 +68,8 @@ struct esth_filter {
     float* R[2] = {nullptr, nullptr};
     uint32_t* sring = nullptr;
     int64_t ready_block = -1;           /* block whose words the RNG stream has been asked for */
-    int64_t main_block = -1;            /* block the main stream has waited for or generated */
+    int64_t rest_block = -1;            /* block whose last words alone it has been asked for */
+    uint64_t main_upto = 0;             /* the main stream has waited for or generated the words of steps below this */
     int64_t inline_block = -1;          /* block generated by the previous step's launch (B = 1) */
     bool inline_rng = false;            /* this filter generates its next step's words inline */
     bool carried = false;               /* ... in shares of all the step's launches (words kept in the same blocks) */
@@ -413,13 +413,13 @@ static uint32_t* status_at(esth_filter* f, uint64_t n) {
     return kk ? status_slot(f, (int)(b & 1), (int)kk) : status_slot(f, (int)((b + 1) & 1), f->B);
 }
 
-/* MTGP words of steps n .. end of n's block, in one launch; the status
- * after each step goes to its slot */
-static int launch_rng(esth_filter* f, uint64_t n, hipStream_t s) {
+/* MTGP words of steps n .. n + steps - 1 of a block, in one launch; the
+ * status after each step goes to its slot */
+static int launch_rng(esth_filter* f, uint64_t n, int steps, hipStream_t s) {
     const uint64_t b = n / f->B;
     const int kk = (int)(n % f->B), p = (int)(b & 1);
     return esth_launch_mtgp(f->e->d_params, status_at(f, n), status_slot(f, p, kk + 1), f->streams, f->K,
-                            step_words(f, n), 1, s, f->B - kk, f->words, (uint64_t)f->K * ESTH_MTGP_N);
+                            step_words(f, n), 1, s, steps, f->words, (uint64_t)f->K * ESTH_MTGP_N);
 }
 
 /* the status between carrier i's share of a step's words and the next one's */
@@ -470,11 +470,15 @@ static int rng_carried(esth_filter* f, bool fused_launch, esth_rng_work* work) {
  * a block the main stream uses the block's words generated inline by the
  * previous step's launch (already in stream order), waits for them
  * (prefetched on the RNG stream), or generates them itself (first step,
- * after a restore, without prefetch).  With `in` (inline_step) the next
- * step's words will be generated by this step's sampling launch and *work
- * receives that launch's MTGP32 work; otherwise, with prefetch on, the next
- * block is generated on the RNG stream while this one's steps run, once the
- * block before this one (whose buffer it reuses) has been consumed. */
+ * after a restore, without prefetch): those up to the end of a pair of steps,
+ * so that this step does not wait for a long block's (a restored filter's
+ * first step with its estimate, the 2M-particle unicycle with 4 landmarks at
+ * the start of a block of 3: 228 us with the block generated whole, 133).  With `in`
+ * (inline_step) the next step's words will be generated by this step's
+ * sampling launch and *work receives that launch's MTGP32 work; otherwise,
+ * with prefetch on, the rest of this block and the next one are generated on
+ * the RNG stream while this one's steps run, once the block before this one
+ * (whose buffer the next one reuses) has been consumed. */
 static int rng_before_step(esth_filter* f, bool in, bool fused_launch, esth_rng_work* work) {
     hipStream_t s = f->stream;
     const uint64_t n = f->steps;
@@ -483,21 +487,21 @@ static int rng_before_step(esth_filter* f, bool in, bool fused_launch, esth_rng_
     *work = esth_rng_work{};
     if (f->carried) return rng_carried(f, fused_launch, work);
     esth_mtgp_inline* mi = &work->mi[ESTH_CARRY_SAMPLE];
-    bool forked = false;
-    if (f->main_block != b) {
+    const uint64_t end = (uint64_t)(b + 1) * f->B;
+    bool cold = false;
+    if (n >= f->main_upto) {
         if (f->inline_block == b) {
-            /* generated by the previous launch on this stream */
-        } else if (f->ready_block == b) {
+            f->main_upto = end;   /* generated by the previous launch on this stream */
+        } else if (f->ready_block == b || f->rest_block == b) {
             ESTH_HIP(hipStreamWaitEvent(s, f->ev_rng_done[p], 0));
+            f->main_upto = end;
         } else {
-            ESTH_TRY(launch_rng(f, n, s));
-            if (f->prefetch && !in) {   /* the next block continues from this block's last status */
-                ESTH_HIP(hipEventRecord(f->ev_fork, s));
-                ESTH_HIP(hipStreamWaitEvent(f->rng_stream, f->ev_fork, 0));
-                forked = true;
-            }
+            const uint64_t pair = (n / ESTH_RNG_BLOCK_DEFAULT + 1) * ESTH_RNG_BLOCK_DEFAULT;
+            const int steps = (int)(std::min(end, pair) - n);
+            ESTH_TRY(launch_rng(f, n, steps, s));
+            f->main_upto = n + steps;
+            cold = true;
         }
-        f->main_block = b;
     }
     if (in) {
         mi->params = f->e->d_params;
@@ -513,15 +517,20 @@ static int rng_before_step(esth_filter* f, bool in, bool fused_launch, esth_rng_
         return ESTH_OK;
     }
     if (f->prefetch && f->ready_block != b + 1) {
-        if (!forked && b > 0) {
-            hipEvent_t e = f->ev_consumed[p ^ 1];
-            if (!f->consumed[p ^ 1]) {   /* the block before generated inline: everything up to here */
-                e = f->ev_fork;
-                ESTH_HIP(hipEventRecord(e, s));
-            }
-            ESTH_HIP(hipStreamWaitEvent(f->rng_stream, e, 0));
+        const bool rest = f->main_upto < end && f->rest_block != b;
+        if (cold || rest || (b > 0 && !f->consumed[p ^ 1])) {
+            /* words follow a status that the main stream left, or a block generated inline: behind everything up to here */
+            ESTH_HIP(hipEventRecord(f->ev_fork, s));
+            ESTH_HIP(hipStreamWaitEvent(f->rng_stream, f->ev_fork, 0));
+        } else if (b > 0) {
+            ESTH_HIP(hipStreamWaitEvent(f->rng_stream, f->ev_consumed[p ^ 1], 0));
         }
-        ESTH_TRY(launch_rng(f, (uint64_t)(b + 1) * f->B, f->rng_stream));
+        if (rest) {
+            ESTH_TRY(launch_rng(f, f->main_upto, (int)(end - f->main_upto), f->rng_stream));
+            ESTH_HIP(hipEventRecord(f->ev_rng_done[p], f->rng_stream));
+            f->rest_block = b;
+        }
+        ESTH_TRY(launch_rng(f, end, f->B, f->rng_stream));
         ESTH_HIP(hipEventRecord(f->ev_rng_done[p ^ 1], f->rng_stream));
         f->ready_block = b + 1;
     }
@@ -999,7 +1008,8 @@ extern "C" int esth_filter_restore(esth_filter* f, const void* buf, size_t bytes
     f->pending = false;
     ESTH_HIP(hipMemcpy(status_at(f, f->steps), p, sizeof(uint32_t) * ESTH_MTGP_N * (size_t)f->K, hipMemcpyHostToDevice));
     f->ready_block = -1;
-    f->main_block = -1;
+    f->rest_block = -1;
+    f->main_upto = 0;
     f->inline_block = -1;
     f->words_upto = 0;
     return ESTH_OK;

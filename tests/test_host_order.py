@@ -145,7 +145,113 @@ def carried_words(ea, fake):
                 assert len({s for s, _ in got}) == 2 and got[-1][1] == block, (m, G, block, got)
 
 
-SCENARIOS = [failed_argmax, failed_batch_step, creation_waits_for_no_stream, carried_words]
+class Order:
+    """Follows a log: which step's words lie where, and what is ordered before what (a clock per stream and for the
+    host).  Words are read after they were written, overwritten after they were read, and every step's words are
+    generated from the status that the step before left."""
+
+    def __init__(self):
+        self.now, self.events, self.host = {}, {}, {}   # stream -> clock (stream -> its count), event -> clock
+        self.status, self.words = {}, {}                # address -> step; address -> [step, writer, readers]
+        self.step = 0
+
+    def restored(self, step):
+        self.status, self.words, self.step = {}, {}, step
+
+    def op(self, s):
+        c = self.now.setdefault(s, {})
+        for k, v in self.host.items():
+            c[k] = max(c.get(k, 0), v)
+        c[s] = c.get(s, 0) + 1
+        return (s, c[s])
+
+    def after(self, s, op):
+        return self.now[s].get(op[0], 0) >= op[1]
+
+    def line(self, l):
+        t = l.split()
+        if t[0] == "hipEventRecord":
+            self.op(t[4])
+            self.events[t[2]] = dict(self.now[t[4]])
+        elif t[0] == "hipStreamWaitEvent":
+            self.op(t[2])
+            for k, v in self.events[t[4]].items():
+                self.now[t[2]][k] = max(self.now[t[2]].get(k, 0), v)
+        elif t[0] == "hipStreamSynchronize":
+            for k, v in self.now.get(t[2], {}).items():
+                self.host[k] = max(self.host.get(k, 0), v)
+        elif t[0] == "launch" and "6k_mtgp" in t[1]:
+            s, n, frm, to, ds, at, dw = t[3], *map(int, t[5:16:2])
+            me = self.op(s)
+            first, by = self.status.get(frm, (self.step, None))
+            assert by is None or self.after(s, by), "the status is not there yet"
+            for i in range(n):
+                old = self.words.get(at + i * dw)
+                assert old is None or all(self.after(s, r) for r in old[2]), f"words of step {old[0]} overwritten"
+                self.words[at + i * dw] = [first + i, me, []]
+                self.status[to + i * ds] = (first + i + 1, me)
+        elif t[0] == "launch" and "k_sample" in t[1]:
+            s = t[3]
+            me = self.op(s)
+            mine = [w for w in self.words.values() if w[0] == self.step]
+            assert mine and all(self.after(s, w[1]) for w in mine), f"words of step {self.step} are not there yet"
+            for w in mine:
+                w[2].append(me)
+            self.step += 1
+
+
+def cold_start(ea, fake):
+    """The first step after a creation or a restore waits for the words of two steps at most, whatever the block, and
+    the others are there in time, from any step on and with prefetch switched off and on."""
+    e = ea.Engine(0)
+    d, p, args = walk(ea, G=3001)
+    for block in (0, 3, 8):
+        if block:
+            os.environ["ESTH_RNG_BLOCK_STEPS"] = str(block)
+        f = ea.Filter(e, d, p)
+        B = f.rng_mode()[1]
+        assert B == (block or 4)
+        f.init_uniform([0.0, 0.0, 0.0])
+        fake.take()
+        o, taken = Order(), 0
+
+        def step():
+            f.step(*args)
+            log = fake.take()
+            for l in log:
+                o.line(l)
+            return log
+
+        snaps = []
+        for k in range(2 * B + 2):
+            ahead = []
+            for l in step():
+                if "k_sample" in l:
+                    break
+                ahead.append(l)
+            if k == 0:
+                assert max(n for _, n in steps_per_block(ahead)[:1]) <= 2, ahead
+            snaps.append(f.snapshot())
+            for l in fake.take():
+                o.line(l)
+        for k, s in enumerate(snaps):
+            for off, on in ((None, None), (1, 2), (1, 3), (2, 4), (3, 4)):
+                f.restore(s)
+                for l in fake.take():
+                    o.line(l)
+                o.restored(k + 1)
+                for i in range(2 * B + 3):
+                    if i in (off, on):
+                        f.set_prefetch(i == on)
+                    log = step()
+                    if i == 0:
+                        main = [l.split()[3] for l in log if "k_sample" in l][0]
+                        assert sum(n for st, n in steps_per_block(log) if st == main) <= 2, log
+        f.close()
+        fake.take()
+
+
+SCENARIOS = [failed_argmax, failed_batch_step, creation_waits_for_no_stream, carried_words, cold_start]
 
 
 @pytest.fixture(scope="session")
