@@ -2432,70 +2432,82 @@ __device__ __forceinline__ void esth_alias_wave(float* __restrict__ st_main, con
     esth_wave_lds_fence();
     uint32_t small_begin = 0, small_end = (uint32_t)nsmall_i;
     const uint64_t below = lane == 0 ? 0ull : (~0ull >> (ESTH_WAVE - lane));
-    for (;;) {
+    /* pairs of the next round: as many as there are small or large items left.
+     * A round makes at most n more items small, so n never grows: rounds of
+     * more than a wave's pairs come first, and those of one pair per lane, the
+     * many of a long chain, have a loop of their own.  They are bound by
+     * latency: a few dependent LDS accesses a round, and the fetch after each
+     * taken branch.  As a branch of the other rounds' loop, two kilobytes from
+     * its head, the same instructions took 193 us in one build and 214 in
+     * another at m = 1024; whole steps now: unicycle10 1024 x 256 257 -> 212
+     * us, unicycle 512 x 4096 with 32 landmarks 167 -> 155. */
+    const auto pairs = [&] {
         const uint32_t a = small_end - small_begin, b = (uint32_t)M - small_end;
-        const uint32_t n = a < b ? a : b;
-        if (n == 0) break;
-        if (n <= (uint32_t)ESTH_WAVE) {   /* the common short round: one pair per lane */
-            const uint32_t k = (uint32_t)lane;
-            const bool act = k < n;
-            uint32_t li = 0;
-            float pL = 0.0f;
-            if (act) {
-                const uint32_t si = sl[small_begin + k];
-                li = sl[small_end + k];
-                const float pS = prob[si];
-                alias[si] = li;
-                pL = (prob[li] + pS) - 1.0f;
+        return a < b ? a : b;
+    };
+    uint32_t n = pairs();
+    if constexpr (M / 2 > ESTH_WAVE) {
+        for (; n > (uint32_t)ESTH_WAVE; n = pairs()) {
+            uint32_t li[J];
+            float pL[J];
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                const uint32_t k = (uint32_t)(j * ESTH_WAVE + lane);
+                li[j] = 0;
+                pL[j] = 0.0f;
+                if (k < n) {
+                    const uint32_t si = sl[small_begin + k];
+                    li[j] = sl[small_end + k];
+                    const float pS = prob[si];
+                    alias[si] = li[j];
+                    pL[j] = (prob[li[j]] + pS) - 1.0f;
+                }
+            }
+            esth_wave_lds_fence();   /* the round's reads before its writes */
+            uint32_t nbs = 0;
+#pragma unroll
+            for (int j = 0; j < J; ++j) {
+                if ((uint32_t)(j * ESTH_WAVE) >= n) break;
+                const uint32_t k = (uint32_t)(j * ESTH_WAVE + lane);
+                const bool act = k < n;
+                const bool bs = act && pL[j] <= 1.0f;
+                const uint64_t bal = __ballot(bs);
+                const uint32_t rs = nbs + (uint32_t)__popcll(bal & below);
+                if (act) {
+                    const uint32_t s2 = bs ? (small_end + rs) : (small_end - 1u + n - (k - rs));
+                    sl[s2] = li[j];
+                    prob[li[j]] = pL[j];
+                }
+                nbs += (uint32_t)__popcll(bal);
             }
             esth_wave_lds_fence();
-            const bool bs = act && pL <= 1.0f;
-            const uint64_t bal = __ballot(bs);
-            const uint32_t rs = (uint32_t)__popcll(bal & below);
-            if (act) {
-                const uint32_t s2 = bs ? (small_end + rs) : (small_end - 1u + n - (k - rs));
-                sl[s2] = li;
-                prob[li] = pL;
-            }
-            esth_wave_lds_fence();
-            small_end += (uint32_t)__popcll(bal);
+            small_end += nbs;
             small_begin += n;
-            continue;
         }
-        uint32_t li[J];
-        float pL[J];
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const uint32_t k = (uint32_t)(j * ESTH_WAVE + lane);
-            li[j] = 0;
-            pL[j] = 0.0f;
-            if (k < n) {
-                const uint32_t si = sl[small_begin + k];
-                li[j] = sl[small_end + k];
-                const float pS = prob[si];
-                alias[si] = li[j];
-                pL[j] = (prob[li[j]] + pS) - 1.0f;
-            }
-        }
-        esth_wave_lds_fence();   /* the round's reads before its writes */
-        uint32_t nbs = 0;
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            if ((uint32_t)(j * ESTH_WAVE) >= n) break;
-            const uint32_t k = (uint32_t)(j * ESTH_WAVE + lane);
-            const bool act = k < n;
-            const bool bs = act && pL[j] <= 1.0f;
-            const uint64_t bal = __ballot(bs);
-            const uint32_t rs = nbs + (uint32_t)__popcll(bal & below);
-            if (act) {
-                const uint32_t s2 = bs ? (small_end + rs) : (small_end - 1u + n - (k - rs));
-                sl[s2] = li[j];
-                prob[li[j]] = pL[j];
-            }
-            nbs += (uint32_t)__popcll(bal);
+    }
+    for (; n != 0; n = pairs()) {   /* one pair per lane */
+        const uint32_t k = (uint32_t)lane;
+        const bool act = k < n;
+        uint32_t li = 0;
+        float pL = 0.0f;
+        if (act) {
+            const uint32_t si = sl[small_begin + k];
+            li = sl[small_end + k];
+            const float pS = prob[si];
+            alias[si] = li;
+            pL = (prob[li] + pS) - 1.0f;
         }
         esth_wave_lds_fence();
-        small_end += nbs;
+        const bool bs = act && pL <= 1.0f;
+        const uint64_t bal = __ballot(bs);
+        const uint32_t rs = (uint32_t)__popcll(bal & below);
+        if (act) {
+            const uint32_t s2 = bs ? (small_end + rs) : (small_end - 1u + n - (k - rs));
+            sl[s2] = li;
+            prob[li] = pL;
+        }
+        esth_wave_lds_fence();
+        small_end += (uint32_t)__popcll(bal);
         small_begin += n;
     }
     if (table_only) {
