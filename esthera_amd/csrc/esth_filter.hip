@@ -20,8 +20,9 @@
  * work-groups (the fused sample+sort at m >= 512, or sample+weight alone) and
  * lasts longer than they need, the next step's words are generated by 96
  * extra work-groups of that launch (inline).  Where the step's launches
- * together last that long (the resampling always has 256-thread work-groups),
- * each of them carries a share of the next step's words (carried).  Neither
+ * together last that long (the resampling has 256-thread work-groups but for
+ * the alias at m = 1024), each of them carries a share of the next step's words
+ * (carried).  Neither
  * needs a second stream or an event, whose waits cost the main stream 10 us
  * at every block of steps.  Otherwise a block of steps' words is generated
  * per launch on a second stream, one block ahead: ESTH_RNG_BLOCK_LONG steps,
@@ -125,57 +126,67 @@ static uint32_t* status_slot(esth_filter* f, int p, int kk) {
     return f->sring + ((size_t)p * (size_t)(f->B + 1) + (size_t)kk) * (size_t)f->K * ESTH_MTGP_N;
 }
 
-/* A launch that carries the next step's MTGP32 work-groups ends no sooner
- * than they do: about 0.5 us per 768-word round of a stream (measured on
- * MI355X beside the sampling), while the sampling itself takes about
- * N (250 + 49 L) / 5.1e13 s for the unicycle with L landmarks (its VALU
- * lane-instructions per particle at the issue rate it sustains).  Inline
- * generation is taken where the sampling is at least 1.25 times longer, so
- * the MTGP32 work-groups hide under it (the 2M-particle unicycle with 32
- * landmarks: 75 against 57 us); elsewhere the words come from the second
- * stream, which overlaps them with the whole step.  Other models have no
- * cost model here and keep the second stream. */
-static bool inline_rng_pays(const esth_filter* f) {
-    if (f->d.model != ESTH_MODEL_UNICYCLE) return false;
-    const int L = ((const esth_unicycle_params*)f->params)->num_landmarks;
-    const double sample_us = (double)f->N * (250.0 + 49.0 * L) / 5.1e13 * 1e6;
-    const double mtgp_us = 0.5 * (double)(f->size / ESTH_MTGP_LARGE);
-    return sample_us >= 1.25 * mtgp_us;
-}
-
-/* The step's launches that can carry MTGP32 work-groups, in stream order, and
- * how long each lasts by itself (us, measured on MI355X: a launch's latency,
- * the sampling's and the sort's VALU lane-instructions per particle at the
- * rate they sustain, the resampling's bytes) */
+/* How long the step's launches last by themselves (us), in stream order, for
+ * the choice of where its words are made: a launch's latency, the sampling's
+ * and the sort's VALU lane-instructions per particle at the rate they sustain,
+ * the resampling's bytes, and the alias resampling's chain of pairings.
+ * Figures of the models in the list, measured on MI355X; a model without one
+ * counts as the lightest, whose launches hide the least. */
 enum { ESTH_CARRY_SAMPLE, ESTH_CARRY_SORT, ESTH_CARRY_RESAMPLE, ESTH_CARRIERS };
-static void carriers(const esth_filter* f, bool fused_launch, double us[ESTH_CARRIERS]) {
-    const double n = (double)f->N;
-    double insts = 800.0;   /* the arms */
-    if (f->d.model == ESTH_MODEL_UNICYCLE) insts = 200.0 + 47.0 * ((const esth_unicycle_params*)f->params)->num_landmarks;
-    else if (f->d.model == ESTH_MODEL_UNICYCLE10) insts = 300.0;
-    else if (f->d.model == ESTH_MODEL_RANDOMWALK3) insts = 130.0;
-    const double sort = 340.0, per_us = 5.1e7, bytes_per_us = 4.0e6, launch = 6.0;
-    us[ESTH_CARRY_SAMPLE] = us[ESTH_CARRY_SORT] = us[ESTH_CARRY_RESAMPLE] = 0.0;
-    if (!fused_launch) {
-        us[ESTH_CARRY_SAMPLE] = launch + n * insts / per_us;
-        if (esth_sort_carries_rng(f->m)) us[ESTH_CARRY_SORT] = launch + n * sort / per_us;
-    } else if (esth_sample_sort_inline_rng(f->m)) {
-        us[ESTH_CARRY_SAMPLE] = launch + n * (insts + sort) / per_us;
+static double sampling_us(const esth_filter* f) {
+    double insts = 130.0;   /* the random walk */
+    switch (f->d.model) {
+    case ESTH_MODEL_UNICYCLE: insts = 200.0 + 47.0 * ((const esth_unicycle_params*)f->params)->num_landmarks; break;
+    case ESTH_MODEL_UNICYCLE10: insts = 300.0; break;
+    case ESTH_MODEL_ROBOTARM5:
+    case ESTH_MODEL_ROBOTARM5_CAMERA:
+    case ESTH_MODEL_DH6: insts = 800.0; break;
+    default: break;
     }
-    if (esth_resample_carries_rng(f->d.resampler, f->m))
-        us[ESTH_CARRY_RESAMPLE] = (launch + n * 8.0 * (f->S + 1) / bytes_per_us) *
-                                  (f->d.resampler == ESTH_RESAMPLE_ALIAS ? 1.4 : 1.0);
+    return (double)f->N * insts / 5.1e7;
 }
-/* a round beside a launch's own work: 0.65 to 0.8 us */
-static double mtgp_us(const esth_filter* f) { return 1.0 + 0.75 * (double)(f->size / ESTH_MTGP_LARGE); }
+static void launches(const esth_filter* f, bool fused_launch, double us[ESTH_CARRIERS]) {
+    const double n = (double)f->N, launch = 6.0, sort = n * 340.0 / 5.1e7;
+    us[ESTH_CARRY_SAMPLE] = launch + sampling_us(f) + (fused_launch ? sort : 0.0);
+    us[ESTH_CARRY_SORT] = fused_launch ? 0.0 : launch + sort;
+    us[ESTH_CARRY_RESAMPLE] = (launch + n * 8.0 * (f->S + 1) / 4.0e6) * (f->d.resampler == ESTH_RESAMPLE_ALIAS ? 1.4 : 1.0);
+}
+/* the same of those that can carry MTGP32 work-groups, 0 for the others */
+static void carriers(const esth_filter* f, bool fused_launch, double us[ESTH_CARRIERS]) {
+    launches(f, fused_launch, us);
+    if (fused_launch && !esth_sample_sort_inline_rng(f->m)) us[ESTH_CARRY_SAMPLE] = 0.0;
+    if (!esth_sort_carries_rng(f->m)) us[ESTH_CARRY_SORT] = 0.0;
+    if (!esth_resample_carries_rng(f->d.resampler, f->m)) us[ESTH_CARRY_RESAMPLE] = 0.0;
+}
+/* A step's words, 768-word rounds of every stream side by side: 0.5 us a round
+ * alone, 0.65 to 0.8 in work-groups beside a launch's own work */
+static double rounds(const esth_filter* f) { return (double)(f->size / ESTH_MTGP_LARGE); }
+static double mtgp_us(const esth_filter* f) { return 1.0 + 0.75 * rounds(f); }
+
+/* The unicycle's sampling launch carries all of the next step's words (inline)
+ * where its sampling alone lasts 0.585 us a round, the sort in the same launch
+ * covering the rest: from 31 landmarks on (40 with the alias).  Around that
+ * line the three ways are within 4 % of each other (26 to 48 landmarks, m = 64,
+ * 512 and 1024, with and without the alias), but inline words bring the
+ * cross-step launch where it applies: 512 x 4096 with 32 landmarks 95 us a step
+ * inline, 101 carried, 102 by the second stream; 512 x 1024 32, 40 and 41.
+ * With few landmarks and many particles they are the slower ones all the same
+ * (512 x 4096 with 8: 71 and 69 us). */
+static bool inline_rng_pays(const esth_filter* f) {
+    return f->d.model == ESTH_MODEL_UNICYCLE && sampling_us(f) >= 0.585 * rounds(f);
+}
 
 /* Carried words cost what the generator's work-groups outlast their launches
- * by, the second stream's about 5.5 us a step: carried up to 4 us of the
- * former.  Measured (whole runs, carried against the second stream): 1024
- * particles 1084 -> 995 us and 4096 1009 -> 924 (32 steps), 256,000 with the
- * alias 1527 -> 1500; where the words take longer than the launches the
- * second stream is the better one (the 2M-particle unicycle with 4 landmarks
- * 14.7 ms against 17.8 carried, the dh6 arm 19.3 against 21.0). */
+ * by, the second stream's an event and a wait at each block of steps: carried
+ * up to 4 us of the former.  Measured on 300 filters of five models, carried
+ * against the second stream in blocks of 4, per step and, in brackets, with the
+ * estimate read after each step, where the host's turn hides words that lie in
+ * the launches but not a wait: randomwalk3 128 x 128 11.7 and 16.8 us, unicycle
+ * 512 x 256 18.7 and 19.2, 512 x 512 23.1 and 22.5, 512 x 1024 32.4 and 28.3
+ * (33.8 and 37.4), 512 x 2048 with 13 landmarks 50.5 and 47.6 (53.2 and 56.8),
+ * randomwalk3 512 x 1024 30.9 and 25.9 (31.6 and 35.5); beyond the line 256 x
+ * 1024 25.5 and 21.4, robotarm5 512 x 512 39.2 and 34.6, 256 x 1024 44.3 and
+ * 30.0.  The line lies between the two uses. */
 static bool carried_rng_pays(const esth_filter* f) {
     double us[ESTH_CARRIERS];
     carriers(f, f->fuse_sample_sort, us);

@@ -251,7 +251,39 @@ def cold_start(ea, fake):
         fake.take()
 
 
-SCENARIOS = [failed_argmax, failed_batch_step, creation_waits_for_no_stream, carried_words, cold_start]
+def words_by_size(ea, fake):
+    """Where a filter's words are made, both sides of each line: the generator's own launches, and the work-groups
+    that the step's launches carry (96 streams)."""
+    def grids(log):
+        names = {"k_sample": "sample", "k_resample": "resample", "k_alias": "resample"}
+        return {v: int(l.split()[5]) for l in log for k, v in names.items() if k in l}
+
+    e = ea.Engine(0)
+    RW, U, S, A = ea.MODEL_RANDOMWALK3, ea.MODEL_UNICYCLE, ea.RESAMPLE_SYSTEMATIC, ea.RESAMPLE_ALIAS
+    for model, m, G, L, res, inline, carriers in (
+            (RW, 512, 256, 0, S, False, "resample"), (RW, 512, 1024, 0, S, False, "sample resample"),
+            (RW, 512, 2048, 0, S, False, ""), (RW, 128, 1024, 0, S, False, "resample"), (RW, 128, 2048, 0, S, False, ""),
+            (U, 512, 512, 20, A, False, "sample resample"), (U, 512, 512, 20, S, False, "sample resample"),
+            (U, 512, 1024, 4, S, False, "sample resample"), (U, 512, 4096, 4, S, False, ""), (U, 512, 4096, 30, S, False, "sample resample"), (U, 512, 4096, 31, S, True, "sample"),
+            (U, 512, 64, 40, S, True, "sample"), (U, 512, 64, 4, S, False, "resample"),
+            (U, 64, 2500, 4, S, False, "sample resample")):
+        p, c, z, _ = ea.randomwalk3_scenario(3, 1) if model == RW else ea.unicycle_scenario(3, L, 20.0, 1)
+        f = ea.Filter(e, ea.filter_desc(model, m=m, G=G, t=1, resampler=res, weights=ea.WEIGHTS_LOG, seed=7), p)
+        f.set_cross_step(False)
+        f.init_uniform([0.0, 0.0, 0.0])
+        for _ in range(3):
+            fake.take()
+            f.step(c[0], z[0], 0.1)
+        carrying, mode = grids(fake.take()), f.rng_mode()[0]
+        f.set_prefetch(False)
+        fake.take()
+        f.step(c[0], z[0], 0.1)
+        alone = grids(fake.take())
+        got = " ".join(n for n in alone if carrying[n] == alone[n] + 96)
+        assert (mode, got) == (inline, carriers), (model, m, G, L, res, carrying, alone)
+
+
+SCENARIOS = [failed_argmax, failed_batch_step, creation_waits_for_no_stream, carried_words, cold_start, words_by_size]
 
 
 @pytest.fixture(scope="session")
