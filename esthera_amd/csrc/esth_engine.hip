@@ -409,18 +409,37 @@ int esth_launch_sort(int S, uint32_t m, float* w, const float* st_in, float* st_
     return ESTH_OK;
 }
 
+/* LDS in addition to the kernel's own for a fused launch that leaves room for a
+ * generator beside it (esth_filter.hip, words_room): at m = 256 at most 9 or 6
+ * work-groups per CU instead of 12, at m = 512 5 or 3 instead of 6, which with
+ * the 160 KB allotted in steps of 1280 bytes always leaves more than the
+ * generator's 3.2 KB.  The dense sort and gather take the LDS pipe from the
+ * generator's chain of dependent LDS reads (0.50 -> 0.55 us a round beside
+ * the arm at m = 512), and where the work-groups fill the LDS to its end the
+ * generator finds no place until one of them ends (robotarm5 256 x 4096: 8
+ * work-groups of 20,480 bytes 83.8 us a step, of 19,200 77.8). */
+template <int LOGM, int S>
+static unsigned room_lds(int room) {
+    const unsigned own = sizeof(float) * ((1 + S) * (1u << LOGM) + esth_sort_floats<LOGM>(0));
+    const unsigned groups = LOGM == 8 ? (room == 1 ? 9 : 6) : LOGM == 9 ? (room == 1 ? 5 : 3) : 0;
+    if (!room || !groups) return 0;
+    const unsigned each = (160u - 10u) * 1024u / groups / 1280u * 1280u;
+    return each > own ? each - own : 0;
+}
+
 template <int MODEL, int L, int LOGM>
 static void launch_sample_sort_m(float* state, uint32_t N, uint32_t G, const float* R, const float* frame,
                                  const esth_frame_arg* fa, int log_w, float* w, int carry, float* st_out,
                                  float2* winner, uint32_t t, float* bt_w, float* bt_s, float* part, const float* gate,
-                                 float keep_thr, int keep_all, const esth_mtgp_inline& mi, hipStream_t s) {
+                                 float keep_thr, int keep_all, int room, const esth_mtgp_inline& mi, hipStream_t s) {
+    const unsigned lds = room_lds<LOGM, esth_model_traits<MODEL>::S>(room);
     if (fa)
         hipLaunchKernelGGL((k_sample_sort<MODEL, L, LOGM, true>), dim3(G + mi.n),
-                           dim3(ESTH_WAVE * esth_ss_waves<LOGM>()), 0, s, state, N, G, R, nullptr, *fa, log_w, w, carry,
+                           dim3(ESTH_WAVE * esth_ss_waves<LOGM>()), lds, s, state, N, G, R, nullptr, *fa, log_w, w, carry,
                            st_out, winner, t, bt_w, bt_s, part, gate, keep_thr, keep_all, mi);
     else
         hipLaunchKernelGGL((k_sample_sort<MODEL, L, LOGM, false>), dim3(G + mi.n),
-                           dim3(ESTH_WAVE * esth_ss_waves<LOGM>()), 0, s, state, N, G, R, frame, esth_frame_arg{},
+                           dim3(ESTH_WAVE * esth_ss_waves<LOGM>()), lds, s, state, N, G, R, frame, esth_frame_arg{},
                            log_w, w, carry, st_out, winner, t, bt_w, bt_s, part, gate, keep_thr, keep_all, mi);
 }
 
@@ -428,10 +447,10 @@ template <int MODEL, int L>
 static int launch_sample_sort_l(int lm, float* state, uint32_t N, uint32_t G, const float* R,
                                 const float* frame, const esth_frame_arg* fa, int log_w, float* w, int carry,
                                 float* st_out, float2* winner, uint32_t t, float* bt_w, float* bt_s, float* part,
-                                const float* gate, float keep_thr, int keep_all, const esth_mtgp_inline& mi,
-                                hipStream_t s) {
+                                const float* gate, float keep_thr, int keep_all, int room,
+                                const esth_mtgp_inline& mi, hipStream_t s) {
 #define ESTH_SS_ARGS state, N, G, R, frame, fa, log_w, w, carry, st_out, winner, t, bt_w, bt_s, part, gate, \
-                     keep_thr, keep_all, mi, s
+                     keep_thr, keep_all, room, mi, s
     switch (lm) {
     case 7: launch_sample_sort_m<MODEL, L, 7>(ESTH_SS_ARGS); break;
     case 8: launch_sample_sort_m<MODEL, L, 8>(ESTH_SS_ARGS); break;
@@ -447,10 +466,10 @@ template <int MODEL>
 static int launch_sample_sort_t(int layout, int lm, float* state, uint32_t N, uint32_t G, const float* R,
                                 const float* frame, const esth_frame_arg* fa, int log_w, float* w, int carry,
                                 float* st_out, float2* winner, uint32_t t, float* bt_w, float* bt_s, float* part,
-                                const float* gate, float keep_thr, int keep_all, const esth_mtgp_inline& mi,
-                                hipStream_t s) {
+                                const float* gate, float keep_thr, int keep_all, int room,
+                                const esth_mtgp_inline& mi, hipStream_t s) {
 #define ESTH_SS_ARGS lm, state, N, G, R, frame, fa, log_w, w, carry, st_out, winner, t, bt_w, bt_s, part, gate, \
-                     keep_thr, keep_all, mi, s
+                     keep_thr, keep_all, room, mi, s
     if (layout == ESTH_LAYOUT_AOS) return launch_sample_sort_l<MODEL, ESTH_LAYOUT_AOS>(ESTH_SS_ARGS);
     if (layout == ESTH_LAYOUT_PACKED) return launch_sample_sort_l<MODEL, ESTH_LAYOUT_PACKED>(ESTH_SS_ARGS);
     return launch_sample_sort_l<MODEL, ESTH_LAYOUT_SOA>(ESTH_SS_ARGS);
@@ -525,7 +544,7 @@ int esth_launch_sample_sort(int model, uint32_t m, float* state, uint32_t N, uin
                             const float* frame, int log_w, float* w, int carry, int layout, float* st_out,
                             float2* winner, uint32_t t, float* bt_w, float* bt_s, float* part, const float* gate,
                             float keep_thr, int keep_all, hipStream_t s, const float* host_frame,
-                            const esth_mtgp_inline* mtgp) {
+                            const esth_mtgp_inline* mtgp, int room) {
     if (!esth_sample_sort_fits(m) || (uint64_t)m * G != N)
         return esth_fail(ESTH_ERR_UNSUPPORTED, "fused sample+sort needs 128 <= m <= 1024 and N = m G");
     const int lm = log2u(m);
@@ -539,7 +558,7 @@ int esth_launch_sample_sort(int model, uint32_t m, float* state, uint32_t N, uin
         fa = &fa_v;
     }
 #define ESTH_SS_ARGS layout, lm, state, N, G, R, frame, fa, log_w, w, carry, st_out, winner, t, bt_w, bt_s, part, \
-                     gate, keep_thr, keep_all, mi, s
+                     gate, keep_thr, keep_all, room, mi, s
     const int rc = esth_with_model(model, [&](auto id) { return launch_sample_sort_t<decltype(id)::value>(ESTH_SS_ARGS); });
 #undef ESTH_SS_ARGS
     if (rc != ESTH_OK) return rc;

@@ -75,6 +75,7 @@ struct esth_filter {
     bool inline_rng = false;            /* this filter generates its next step's words inline */
     bool carried = false;               /* ... in shares of all the step's launches (words kept in the same blocks) */
     uint64_t words_upto = 0;            /* carried: steps below this have their words */
+    int words_room = 0;                 /* room that the fused launch leaves the second stream's words */
     bool prefetch = true;
     bool fuse_sample_sort = false;      /* sample+weight and sort in one launch (k_sample_sort) */
     hipEvent_t ev_rng_done[2], ev_consumed[2], ev_fork;
@@ -194,6 +195,26 @@ static bool carried_rng_pays(const esth_filter* f) {
            mtgp_us(f) <= us[ESTH_CARRY_SAMPLE] + us[ESTH_CARRY_SORT] + us[ESTH_CARRY_RESAMPLE] + 4.0;
 }
 
+/* Where the second stream's words (0.5 us a round by themselves) outlast the
+ * step's launches, they bound the step, and the fused launch of models of many
+ * dimensions leaves them room (esth_engine.hip, room_lds): some where they last
+ * 1.15 times as long, more from 1.33 on, where the launches have the time.  Per
+ * step, and in brackets with the estimate read after each, where the launches'
+ * own time counts too; without, with some, with more room: robotarm5 256 x 4096
+ * (1.28) 82.7 (79.2), 77.7 (81.8), 75.3 us (84.6); 512 x 2048 80.6 (71.6), 76.8
+ * (73.0), 73.7 (78.8); 256 x 6144 (1.37) 122 (112), 115 (110), 110 (109); 512 x
+ * 4096 (1.42) 157 (149), 152 (151), 147 (144).  Below 1.15 the launches bound
+ * the step and only lose by it (256 x 2048, more room: 42 -> 46), as do those
+ * of three dimensions, short of waves then, at any size (randomwalk3 512 x 4096
+ * 62 -> 69, unicycle 512 x 8192 118 -> 148). */
+static int words_room(const esth_filter* f) {
+    if (f->inline_rng || f->carried || f->S < 9) return 0;
+    double us[ESTH_CARRIERS];
+    launches(f, true, us);
+    const double ratio = (1.0 + 0.5 * rounds(f)) / (us[ESTH_CARRY_SAMPLE] + us[ESTH_CARRY_RESAMPLE]);
+    return ratio >= 1.33 ? 2 : ratio >= 1.15 ? 1 : 0;
+}
+
 /* words of each stream that each launch generates: all in the resampling
  * where it lasts that long, else in proportion to what the launches last */
 static void carried_shares(const esth_filter* f, bool fused_launch, uint32_t words[ESTH_CARRIERS]) {
@@ -276,6 +297,7 @@ extern "C" int esth_filter_create(esth_engine* e, const esth_filter_desc* d, con
         if (v >= 1 && v <= ESTH_RNG_BLOCK) blk = (uint64_t)v;
     }
     f->carried = !f->inline_rng && blk == 0 && carried_rng_pays(f);
+    f->words_room = words_room(f);
     const uint64_t two = 2ull * sizeof(float) * f->words;   /* two blocks of one step */
     if (blk == 0)
         blk = f->inline_rng ? 1
@@ -593,7 +615,7 @@ static int enqueue_sample(esth_filter* f, uint64_t n, const float* d_frame, cons
         const float keep_thr = carry ? INFINITY : d.resampling_threshold;
         ESTH_TRY(esth_launch_sample_sort(d.model, f->m, f->state, N, f->G, R, d_frame, log_w, f->w, d.carry_weights,
                                          d.state_layout, f->tmp, x.winner, f->t, x.bt_w, x.bt_s, x.part,
-                                         R + (size_t)N * f->V + N, keep_thr, keep_all, s, h_frame, mi));
+                                         R + (size_t)N * f->V + N, keep_thr, keep_all, s, h_frame, mi, f->words_room));
         if (timing) ESTH_HIP(hipEventRecord(ev[2], s));
     } else {
         /* sampling_importance with Box-Muller fused (pf_generic.c:521-533) */

@@ -123,11 +123,12 @@ int esth_launch_kb_sample_sort(int model, int S, int lm, const esth_bfilter* F, 
                                hipStream_t st);
 bool esth_sample_sort_fits(uint32_t m);
 bool esth_sample_sort_pays(int model, int layout, uint32_t m);   /* fits, and costs the sampling no occupancy */
+/* room (0, 1, 2): fewer work-groups per CU, with LDS left for a generator on another stream (m = 256 and 512) */
 int esth_launch_sample_sort(int model, uint32_t m, float* state, uint32_t N, uint32_t G, const float* R,
                             const float* frame, int log_w, float* w, int carry, int layout, float* st_out,
                             float2* winner, uint32_t t, float* bt_w, float* bt_s, float* part, const float* gate,
                             float keep_thr, int keep_all, hipStream_t s,
-                            const float* host_frame = nullptr, const esth_mtgp_inline* mtgp = nullptr);
+                            const float* host_frame = nullptr, const esth_mtgp_inline* mtgp = nullptr, int room = 0);
 /* whether esth_launch_sample_sort can carry MTGP32 work-groups at this m */
 bool esth_sample_sort_inline_rng(uint32_t m);
 /* publish: result is followed by the argmaxes' count, est as long as

@@ -57,13 +57,13 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* sh, hipStream_t* 
     *g = g_grid, *b = g_block, *sh = g_shmem, *s = g_stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t, hipStream_t s) {
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t lds, hipStream_t s) {
     const std::string& name = g_kernels[f];
     if (name.find("6k_mtgp") != std::string::npos)   /* words and statuses of its steps: addresses and strides in bytes */
         return say("launch %s stream %d steps %d from %zu to %zu stride %llu words %zu stride %llu", name.c_str(), id(s),
                    *(int*)args[8], *(size_t*)args[2], *(size_t*)args[3], 4ull * *(uint64_t*)args[10], *(size_t*)args[6],
                    4ull * *(uint64_t*)args[9]);
-    return say("launch %s stream %d grid %u", name.c_str(), id(s), grid.x);
+    return say("launch %s stream %d grid %u lds %zu", name.c_str(), id(s), grid.x, lds);
 }
 hipError_t hipGetLastError() {
     const hipError_t e = g_last;

@@ -283,7 +283,39 @@ def words_by_size(ea, fake):
         assert (mode, got) == (inline, carriers), (model, m, G, L, res, carrying, alone)
 
 
-SCENARIOS = [failed_argmax, failed_batch_step, creation_waits_for_no_stream, carried_words, cold_start, words_by_size]
+def room_for_the_words(ea, fake):
+    """Where the second stream's words bound an arm's step, the fused launch leaves them LDS on every CU: the
+    work-groups that fit into its 160 KB, allotted in steps of 1280 bytes, are so many and leave the generator's 3200."""
+    e = ea.Engine(0)
+    for model, m, G, L, room in (("ROBOTARM5", 512, 4096, 0, 3), ("ROBOTARM5", 512, 2048, 0, 5), ("ROBOTARM5", 256, 4096, 0, 9),
+                                 ("ROBOTARM5", 256, 8192, 0, 6), ("ROBOTARM5", 1024, 2048, 0, 0), ("ROBOTARM5", 512, 1024, 0, 0),
+                                 ("ROBOTARM5", 256, 2048, 0, 0), ("ROBOTARM5", 512, 64, 0, 0), ("ROBOTARM5", 128, 8192, 0, 0),
+                                 ("DH6", 512, 2048, 0, 0), ("UNICYCLE", 512, 4096, 4, 0), ("RANDOMWALK3", 512, 4096, 0, 0)):
+        if model == "ROBOTARM5":
+            p, c, z = None, ea.RobotArm5Control(), ea.RobotArm5Measurement()
+        elif model == "DH6":
+            (p, zs, _), c = ea.dh6_scenario(3, 1), ea.DH6Control()
+            z = zs[0]
+        else:
+            p, cs, zs, _ = ea.randomwalk3_scenario(3, 1) if model == "RANDOMWALK3" else ea.unicycle_scenario(3, L, 20.0, 1)
+            c, z = cs[0], zs[0]
+        S = ea.STATE_DIM[getattr(ea, "MODEL_" + model)]
+        f = ea.Filter(e, ea.filter_desc(getattr(ea, "MODEL_" + model), m=m, G=G, t=1, resampler=ea.RESAMPLE_SYSTEMATIC,
+                                        weights=ea.WEIGHTS_LOG), p)
+        f.init_uniform([0.0] * S)
+        fake.take()
+        f.step(c, z, 0.1)
+        lds = [int(l.split()[7]) for l in fake.take() if "k_sample_sort" in l]
+        f.close()
+        assert len(lds) == 1 and (lds[0] > 0) == (room > 0), (model, m, G, lds)
+        if room:
+            own = 4 * ((1 + S) * m + 2 * (m + 64)) + lds[0]
+            each = -(-own // 1280) * 1280
+            assert 163840 // each == room and own <= 65536 and 163840 - room * each >= 3200
+
+
+SCENARIOS = [failed_argmax, failed_batch_step, creation_waits_for_no_stream, carried_words, cold_start, words_by_size,
+             room_for_the_words]
 
 
 @pytest.fixture(scope="session")
