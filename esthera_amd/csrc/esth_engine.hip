@@ -690,11 +690,13 @@ static void launch_resample_argmax_t(float* st_main, const float* st_tmp, const 
      * sub-filters' CDFs and staged planes fit in 48 KB of LDS (at m = 256 in
      * the batched classes the halves were too short to pay for the barriers).
      * Where they do not fit, four waves while the sub-filters are few: one
-     * wave each is then a long chain on a chip mostly idle (robotarm5 at m =
-     * 1024, whole steps, one wave against four: 8 sub-filters 34.6 and 25.3
-     * us, 500 52.2 and 43.6 (the launch 28 and 16), 768 60.1 and 58.6, 1024
-     * 117.1 and 118.7; dh6 at 512: 8 22.3 and 18.6, 256 28.6 and 26.5, 500
-     * 35.2 and 38.4; at 1024: 512 72.5 and 68.0).  For the smaller ones the
+     * wave each is then a long chain on a chip mostly idle.  Whole steps, one
+     * wave against four, nine planes (robotarm5) at m = 1024: 8 sub-filters
+     * 34.6 and 25.3 us, 256 50.9 and 41.4, 512 56.4 and 46.6, 768 63.6 and 61.4,
+     * 1024 80.9 and 80.1; twelve (dh6): 256 69.1 and 56.2, 512 73.0 and 69.0,
+     * 640 78.4 and 74.2, 768 90.6 and 90.4, 1024 97.9 and 98.4; twelve at m =
+     * 512: 64 24.2 and 20.0, 256 28.9 and 26.1, 384 33.4 and 32.8, 512 35.7 and
+     * 38.5.  For the smaller ones the
      * wave counts are even or worse (unicycle and robotarm5 at m = 256 with
      * two waves 0-5 % slower, at 512 with four -1 to +4 %). */
     constexpr bool halves = LOGM >= 9 && (1 + S) * (1 << LOGM) <= 6144;

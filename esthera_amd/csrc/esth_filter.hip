@@ -310,9 +310,15 @@ extern "C" int esth_filter_create(esth_engine* e, const esth_filter_desc* d, con
                (d->topology == ESTH_TOPO_RING || d->topology == ESTH_TOPO_TORUS) && !d->carry_weights &&
                d->state_layout == ESTH_LAYOUT_SOA;
     for (int i = 0; i < 7; ++i) hipEventCreate(&f->ev[i]);
-    /* these order launches of one device: no system-scope write-back at each
-     * (4 landmarks, 2M particles 14.83 -> 14.54 ms, dh6 18.77 -> 18.52, two
-     * events per block of 2 steps) */
+    /* These order launches of one device.  Without the system fence an event
+     * does not make memory visible to the host and to other devices (neither
+     * reads the words or statuses); launches of this device see what those
+     * before them wrote by their own release and acquire, as on one stream.
+     * With the fence, whole runs of 200 steps with two events per block of 2:
+     * 4 landmarks, 2M particles 14.83 -> 14.54 ms, dh6 18.77 -> 18.52; with a
+     * device-scope release in its place (hipEventReleaseToDevice) steps are 1
+     * to 4 % longer (randomwalk3 128 x 3001 24.2 and 24.8 us, unicycle 512 x
+     * 2048 38.1 and 39.6). */
     for (int i = 0; i < 2; ++i) {
         hipEventCreateWithFlags(&f->ev_rng_done[i], hipEventDisableTiming | hipEventDisableSystemFence);
         hipEventCreateWithFlags(&f->ev_consumed[i], hipEventDisableTiming | hipEventDisableSystemFence);

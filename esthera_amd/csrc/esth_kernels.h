@@ -688,12 +688,6 @@ __host__ __device__ constexpr int esth_sort_floats(int least) {
     return n > least ? n : least;
 }
 
-/* whether the work-group's other waves stay for the planes after the sort */
-template <int LOGM, int S>
-__host__ __device__ constexpr bool esth_sort_shared() {
-    return esth_sort_packed<LOGM>();
-}
-
 /* where a lane's value r lies when the register's bits are [B, B + LOGE) of
  * the position (the lane's low B bits below them, its others above):
  * esth_sort_slot(lane) + esth_sort_step(r) */
@@ -1048,11 +1042,12 @@ __device__ __forceinline__ void esth_store_plane_run(float* __restrict__ st, int
     for (int r = 0; r < E; ++r) st[b + (size_t)r * stride] = v[r];
 }
 
-/* stage_w: this wave's LDS, esth_sort_floats (or, not FROM_LDS, at least its
- * sub-filters' positions), 8-byte aligned.
- * FROM_LDS: the sub-filter's weights and planes are already in LDS at `src`
- * (src[0..M) the weights, src[(1 + c) M ..) plane c): the keys are read from
- * there and the gather permutes there, with no global reads */
+/* stage_w: this wave's LDS, esth_sort_floats and at least its sub-filters'
+ * positions, 8-byte aligned (not FROM_LDS).
+ * FROM_LDS (two positions per lane, so not the packed sort): the sub-filter's
+ * weights and planes are already in LDS at `src` (src[0..M) the weights,
+ * src[(1 + c) M ..) plane c): the keys are read from there and the gather
+ * permutes there, with no global reads */
 /* v[r] to particle i0 + r * stride of plane c (a strided run: with stride
  * 64, each r is one coalesced store across the wave) */
 template <int E, int S>
@@ -1078,7 +1073,7 @@ __device__ __forceinline__ void esth_sort_sub(float* __restrict__ w, const float
     using TL = esth_tile<LOGM, LANES>;
     constexpr int M = TL::M, E = TL::E, LPS = TL::LPS;
     constexpr bool PACKED = esth_sort_packed<LOGM, LANES>();
-    static_assert(!FROM_LDS || M >= ESTH_WAVE, "an LDS-resident sub-filter of at least one wave's positions");
+    static_assert(!FROM_LDS || (M >= ESTH_WAVE && !PACKED), "an LDS-resident sub-filter of one or two positions per lane");
     const int lane = threadIdx.x & (ESTH_WAVE - 1);
     const int le = (lane % LPS) * E;
     float* stage = FROM_LDS ? nullptr : stage_w + (lane - lane % LPS) * E;   /* this sub-filter's M floats */
@@ -1359,13 +1354,13 @@ __global__ __launch_bounds__(ESTH_WAVE * esth_ss_waves<LOGM>()) void k_sample_so
         for (int c = 0; c < S; ++c) *reinterpret_cast<float2*>(sub + (1 + c) * M + q) = make_float2(s0[c], s1[c]);
     }
     __syncthreads();
-    if constexpr (esth_sort_shared<LOGM, S>()) {
+    if constexpr (esth_sort_packed<LOGM>()) {   /* the other waves stay for the planes */
         esth_sort_group<LOGM, S, esth_ss_waves<LOGM>()>(w, st_out, N, G, g, winner, t, bt_w, bt_s, part, log_w, sub,
                                                         sub + (1 + S) * M);
     } else {
         if (threadIdx.x >= ESTH_WAVE) return;
         esth_sort_sub<LOGM, S, false, true>(w, nullptr, st_out, N, G, g, true, winner, nullptr, t, bt_w, bt_s, part,
-                                            log_w, sub + (1 + S) * M, ESTH_LAYOUT_SOA, sub);
+                                            log_w, nullptr, ESTH_LAYOUT_SOA, sub);
     }
 }
 
@@ -1415,7 +1410,7 @@ static __global__ void k_exchange(float* __restrict__ st, float* __restrict__ w,
  * previous one.  A round is one pass over the candidates (held in registers
  * up to 8 per thread) and a tree over the 1024 threads' best: the tree's
  * levels 512 .. 64 apart in the first wave's registers, the others by lane
- * exchanges, two barriers a round.  Bound by latency (2000 candidates, 4
+ * exchanges, three barriers a round.  Bound by latency (2000 candidates, 4
  * rounds: 11.6 -> 9.9 us).  sw, si: 1024 words of LDS each. */
 struct esth_cand {
     float w;
@@ -2052,13 +2047,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
         for (int c = 0; c < S; ++c) *reinterpret_cast<float2*>(sub + (1 + c) * M + q) = make_float2(s0[c], s1[c]);
     }
     __syncthreads();
-    if constexpr (esth_sort_shared<LOGM, S>()) {
-        esth_sort_group<LOGM, S, 4>(w, tmp, N, G, g, winner_k1, xk.t, bt_w_k1, bt_s_k1, part_k1, log_w, sub, res);
-    } else {
-        if (threadIdx.x >= ESTH_WAVE) return;
-        esth_sort_sub<LOGM, S, false, true>(w, nullptr, tmp, N, G, g, true, winner_k1, nullptr, xk.t, bt_w_k1,
-                                            bt_s_k1, part_k1, log_w, res, ESTH_LAYOUT_SOA, sub);
-    }
+    esth_sort_group<LOGM, S, 4>(w, tmp, N, G, g, winner_k1, xk.t, bt_w_k1, bt_s_k1, part_k1, log_w, sub, res);
 }
 
 /* =========================================================== Vose alias
@@ -2708,13 +2697,13 @@ __attribute__((amdgpu_waves_per_eu(esth_kbss_waves_per_eu<MODEL>()))) void kb_sa
         for (int c = 0; c < S; ++c) *reinterpret_cast<float2*>(lds + (1 + c) * M + q) = make_float2(s0[c], s1[c]);
     }
     __syncthreads();
-    if constexpr (esth_sort_shared<LOGM, S>()) {
+    if constexpr (esth_sort_packed<LOGM>()) {   /* the other waves stay for the planes */
         esth_sort_group<LOGM, S, esth_ss_waves<LOGM>()>(f.w, f.tmp, f.N, f.G, e.y, (float2*)f.winner, f.t, f.bt_w,
                                                         f.bt_s, f.part, log_w, lds, lds + (1 + S) * M);
     } else {
         if (threadIdx.x >= ESTH_WAVE) return;
         esth_sort_sub<LOGM, S, false, true>(f.w, nullptr, f.tmp, f.N, f.G, e.y, true, (float2*)f.winner, nullptr, f.t,
-                                            f.bt_w, f.bt_s, f.part, log_w, lds + (1 + S) * M, ESTH_LAYOUT_SOA, lds);
+                                            f.bt_w, f.bt_s, f.part, log_w, nullptr, ESTH_LAYOUT_SOA, lds);
     }
 }
 
