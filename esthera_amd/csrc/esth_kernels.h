@@ -12,10 +12,10 @@
  * Execution model: one 64-lane wave per sub-filter for sort and resampling
  * (E = m/64 elements per lane, lane-major, e = lane*E + r; for m < 64 a wave
  * holds 64/m sub-filters with one element per lane).  Strides below E are
- * register compare-exchanges, larger ones cross lanes by xor shuffles, so the
- * sort needs no LDS and no barrier.  Vose's alias build keeps the reference's
- * work-group-per-sub-filter shape because its pairing rounds are
- * data-dependent and share worklists.
+ * register compare-exchanges; larger ones cross lanes by exchanges, for m >=
+ * 256 the widest by trades through the wave's own LDS; the sort has no
+ * barrier.  Vose's alias build runs on one wave per sub-filter from m = 64 on;
+ * below it keeps the reference's work-group per sub-filter.
  */
 #ifndef ESTH_KERNELS_H
 #define ESTH_KERNELS_H
@@ -27,6 +27,16 @@
 #include "esth_models.h"
 
 #define ESTH_WAVE 64
+
+/* where a step's large kernels start.  Two of them that alternate pass the 64
+ * KB instruction cache of two CUs (dh6 at m = 512: 33 KB of sampling and sort,
+ * 51 of resampling), and how much of one outlives the other depends on where
+ * their code lies in its sets: with the default of 256 bytes every change of
+ * another kernel's size moved them (dh6 512 x 1536 47.6 to 51.6 us a step in
+ * builds of the same kernels, 500 sub-filters of the arm at m = 1024 47.0 and
+ * 47.8).  Starts at multiples of 512, 1024, 2048, 4096 and 8192: 49.0, 48.5,
+ * 48.3, 51.8 and 50.6 us; 512 x 512 35.2, 35.0, 35.4, 35.3 and 35.4. */
+#define ESTH_KERNEL_ALIGN __attribute__((aligned(1024)))
 
 /* ------------------------------------------------------------ wave ops */
 __device__ __forceinline__ float esth_shfl_xor(float v, int mask) {
@@ -194,6 +204,7 @@ __device__ __forceinline__ void esth_mtgp_wg(const uint32_t* __restrict__ params
 /* streams j = blockIdx.x, blockIdx.x + gridDim.x, ...: a launch over many
  * short streams (a batch's per-filter streams) keeps a resident grid instead
  * of one work-group launch per stream */
+ESTH_KERNEL_ALIGN
 static __global__ __launch_bounds__(256) void k_mtgp(const uint32_t* __restrict__ params, uint32_t mask,
                                               const uint32_t* status_in, uint32_t* status_out,
                                               const esth_mtgp_stream* __restrict__ streams, uint32_t nstreams,
@@ -1261,6 +1272,7 @@ __device__ __forceinline__ void esth_sort_group(float* __restrict__ w, float* __
 }
 
 template <int LOGM, int S>
+ESTH_KERNEL_ALIGN
 __global__ __launch_bounds__(256) void k_sort(float* __restrict__ w, const float* __restrict__ st_in,
                                               float* __restrict__ st_out, uint32_t N, uint32_t G,
                                               float2* __restrict__ winner, int* __restrict__ perm,
@@ -1302,6 +1314,7 @@ __host__ __device__ constexpr int esth_ss_waves() {
  * data-dependent alias gate, always (keep_all).  The sort's wave runs beside
  * other work-groups' sampling instead of after all of them. */
 template <int MODEL, int L, int LOGM, bool FA>
+ESTH_KERNEL_ALIGN
 __global__ __launch_bounds__(ESTH_WAVE * esth_ss_waves<LOGM>()) void k_sample_sort(float* __restrict__ state, uint32_t N,
                                                                  uint32_t G, const float* __restrict__ R,
                                                                  const float* __restrict__ frame_ptr,
@@ -1733,6 +1746,7 @@ __global__ __launch_bounds__(256) void k_resample(float* __restrict__ st_main,
  * reads, so one launch does both and the argmax's single work-group runs in
  * the shadow of the resampling instead of on its own before the exchange. */
 template <int LOGM, int S>
+ESTH_KERNEL_ALIGN
 __global__ __launch_bounds__(256) void k_resample_argmax(float* __restrict__ st_main,
                                                          const float* __restrict__ st_tmp,
                                                          const float* w,
@@ -1939,6 +1953,7 @@ __device__ __forceinline__ void esth_resample_sub2(float* __restrict__ st_main, 
  * instead of m / 64: 73 registers for nine planes at m = 1024 instead of 188,
  * and a chain a third as long (500 sub-filters 28 -> 16 us; bytes alone 8) */
 template <int LOGM, int S, int W>
+ESTH_KERNEL_ALIGN
 __global__ __launch_bounds__(256) void k_resample2_argmax(float* __restrict__ st_main,
                                                           const float* __restrict__ st_tmp, const float* w,
                                                           const float* __restrict__ rnd, uint32_t N, uint32_t G,
@@ -1984,6 +1999,7 @@ __global__ __launch_bounds__(256) void k_resample2_argmax(float* __restrict__ st
  * then rewritten by its own work-group only.  For the scan resamplers on a
  * ring or torus with t > 0, SOA state and no carried weights. */
 template <int MODEL, int LOGM, bool FA>
+ESTH_KERNEL_ALIGN
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_step_x(
     float* tmp, float* w, const float* __restrict__ rnd_k, float thr, int systematic, const esth_xch xk,
     const float2* __restrict__ winner_k, const float* __restrict__ part_k, const float* __restrict__ best_k,
@@ -2571,6 +2587,7 @@ __global__ __launch_bounds__(256) void k_alias_w(float* __restrict__ st_main, co
  * copy, the resampling the weights, uniforms, sorted state and best-t copy;
  * neither writes what the other reads. */
 template <int LOGM, int S>
+ESTH_KERNEL_ALIGN
 __global__ __launch_bounds__(256) void k_alias_argmax_w(float* __restrict__ st_main, const float* __restrict__ st_tmp,
                                                         const float* w, const float* __restrict__ rnd, uint32_t N,
                                                         uint32_t G, float thr, int adaptive, int log_w,
