@@ -285,7 +285,8 @@ int esth_filter_init(esth_filter* f, const float* state_soa);
  * control/measurement are the model's structs (copied before return). */
 int esth_filter_step(esth_filter* f, const void* control, const void* measurement, float dt);
 int esth_filter_sync(esth_filter* f);
-/* Estimate of the last step (waits for it, not for the step's resampling). */
+/* Estimate of the last step (waits for it, not for the step's resampling;
+ * ESTH_ERR_DEVICE if the device never wrote it). */
 int esth_filter_estimate(esth_filter* f, esth_estimate* out);
 /* Current particles (state_dim planes of m*G floats) and per-particle
  * weights as left by the sort/exchange stages (sorted per sub-filter). */
